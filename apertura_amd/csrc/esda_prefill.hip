@@ -569,33 +569,74 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
     }
 }
 
-// out(i, h, 4 dims) = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the splits
-// with l_s > 0 (one thread per (row, 4 dims)).
+// out(i, h, :) = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the splits with
+// l_s > 0.  One wave per (row, 64 * VEC dims): lane j first loads (m, l) of split j (and
+// j + 64, ..), so the max, the weights and the denominator take one round trip and wave
+// reductions; the wave then walks the live splits (a ballot: wave-uniform, so an empty
+// split costs nothing) with MB of their partial rows in flight.
+// Memory-bound: splits * D * 4 bytes per row, read once.  A thread per 4 dims walking the
+// splits one after another was bound by their latency instead (512 rows of D = 512: 20
+// splits took 17 us; MERGE_AFTER).
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
+    constexpr int VEC = D >= 256 ? 4 : D / 64;  // dims per lane
+    constexpr int PARTS = D / (64 * VEC);       // waves per row
+    constexpr int MB = 8;                       // partial rows in flight
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const int lane = threadIdx.x & 63;
     const long long nrows = (long long) p.Sq * p.Hq;
-    const long long t = (long long) blockIdx.x * 256 + threadIdx.x;
-    if (t >= nrows * (D / 4)) return;
-    const long long row = t / (D / 4);
-    const int d4 = (int) (t % (D / 4));
-    float M = -INFINITY;
-    for (int s = 0; s < p.splits; ++s) {
-        const f32x2 ml = *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row));
-        if (ml[1] > 0.0f) M = fmaxf(M, ml[0]);
+    const long long wv = (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+    if (wv >= nrows * PARTS) return;
+    const long long row = wv / PARTS;
+    const int d0 = (int) (wv % PARTS) * 64 * VEC + lane * VEC;
+    auto ml_of = [&](int s) {
+        return s < p.splits ? *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row))
+                            : f32x2{-INFINITY, 0.0f};
+    };
+    f32x2 ml = ml_of(lane);
+    float M = ml[1] > 0.0f ? ml[0] : -INFINITY;
+    for (int s = lane + 64; s < p.splits; s += 64) {
+        const f32x2 x = ml_of(s);
+        if (x[1] > 0.0f) M = fmaxf(M, x[0]);
     }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
     float den = 0.0f;
-    f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < p.splits; ++s) {
-        const f32x2 ml = *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row));
-        if (!(ml[1] > 0.0f)) continue;
-        const float w = __builtin_amdgcn_exp2f(ml[0] - M);
-        den += ml[1] * w;
-        num += w * *reinterpret_cast<const f32x4 *>(p.part_acc + ((long long) s * nrows + row) * D + 4 * d4);
+    vec num = 0.0f;
+    const float *acc = p.part_acc + row * D + d0;
+    const long long ss = nrows * D;
+    for (int s0 = 0; s0 < p.splits; s0 += 64) {
+        if (s0) ml = ml_of(s0 + lane);
+        const float w = ml[1] > 0.0f ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.0f;
+        den += ml[1] > 0.0f ? ml[1] * w : 0.0f;
+        unsigned long long live = __builtin_amdgcn_ballot_w64(ml[1] > 0.0f);
+        while (live) {
+            vec a[MB];
+            float wj[MB];
+            int n = 0;
+#pragma unroll
+            for (int j = 0; j < MB; ++j)
+                if (live) {
+                    const int b = __builtin_ctzll(live);
+                    live &= live - 1;
+                    wj[j] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), b));
+                    a[j] = *reinterpret_cast<const vec *>(acc + (s0 + b) * ss);
+                    n = j + 1;
+                }
+#pragma unroll
+            for (int j = 0; j < MB; ++j)
+                if (j < n) num += wj[j] * a[j];
+        }
     }
-    const f32x4 v4 = num * (1.0f / den);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) den += __shfl_xor(den, o);
+    const vec v = num * (1.0f / den);
+    typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
+    bvec b;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) b[e] = (__bf16) v[e];
     const int i = (int) (row / p.Hq), h = (int) (row % p.Hq);
-    bf16x4 b4 = {(__bf16) v4[0], (__bf16) v4[1], (__bf16) v4[2], (__bf16) v4[3]};
-    *reinterpret_cast<bf16x4 *>(p.out + (size_t) i * p.o_rs + (size_t) h * p.o_hs + 4 * d4) = b4;
+    *reinterpret_cast<bvec *>(p.out + (size_t) i * p.o_rs + (size_t) h * p.o_hs + d0) = b;
 }
 
 // ------------------------------------------------------------ raw-K reconstruction
@@ -836,8 +877,8 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
             hipLaunchKernelGGL((prefill_kernel<256, 1>), grid, block, 0, st, p);
     }
     if ((stages & 2) && p.splits > 1) {
-        const long long n = (long long) p.Sq * p.Hq * (D / 4);
-        hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, p);
+        const long long waves = (long long) p.Sq * p.Hq * (D >= 256 ? D / 256 : 1);
+        hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st, p);
     }
 }
 
