@@ -91,7 +91,7 @@ __host__ __device__ inline void tile_keys(const PrefillParams &p, int tile, int 
 // Eight waves per workgroup (two per SIMD) and QB 16-query blocks per wave.  O^T takes
 // QB * D / 16 accumulator registers per lane beside Q^T's QB * D / 8 and 8 QB of scores,
 // within the 256 registers of two waves per SIMD: QB = 1 at D = 512 (two blocks do not
-// fit without spills), 1 or 2 at D = 256 (pick_qb), 2 at D = 128.  (Measured: at D = 256,
+// fit without spills), 1 or 2 at D = 256 (kTilings256), 2 at D = 128.  (Measured: at D = 256,
 // four waves of two blocks -- one wave per SIMD -- ran 6% slower than eight waves of one
 // block, and forming the next stage's scores during this stage's softmax -- a second set
 // of score registers, forcing one block per wave at D = 256 -- was 5-20% slower.)
@@ -100,7 +100,7 @@ __host__ __device__ inline void tile_keys(const PrefillParams &p, int tile, int 
 // block and take the even and the odd stages of the tile's keys, over a ring of four
 // stages per tensor (132 KB), and fold their (m, l, O^T) together through LDS at the end.
 // A tile is then 64 query rows, so a chunk whose 128-row tiles would leave CUs idle gets
-// twice the tiles instead of key splits -- no fp32 partials and no merge launch -- while
+// twice the tiles before any key split -- no fp32 partials and no merge launch -- while
 // each wave's work per stage and the barriers per stage stay those of the plain kernel.
 constexpr int kWaves = 8;
 #ifndef PV_DEPTH
@@ -575,8 +575,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
 // reductions; the wave then walks the live splits (a ballot: wave-uniform, so an empty
 // split costs nothing) with MB of their partial rows in flight.
 // Memory-bound: splits * D * 4 bytes per row, read once.  A thread per 4 dims walking the
-// splits one after another was bound by their latency instead (512 rows of D = 512: 20
-// splits took 17 us; MERGE_AFTER).
+// splits one after another was bound by their latency instead: 512 rows of D = 512 with 18
+// splits 8.2 us against 4.3 here, with 32 splits 19.9 against 6.3.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     constexpr int VEC = D >= 256 ? 4 : D / 64;  // dims per lane
@@ -761,23 +761,48 @@ int fail(int code, const std::string &msg) {
 
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
-// 16-query blocks per wave: two where they fit the registers (D <= 256), except at
-// D = 256 when the two-block tiles would leave CUs idle without key splits -- a split's
-// partials cost 4 D bytes per query row written and read again.
-int pick_qb(int D, long long rows, int Hkv) {
-    if (D == 512) return 1;
-    if (D == 128) return 2;
-    const long long tiles2 = (rows + 16 * 2 * kWaves - 1) / (16 * 2 * kWaves);
-    return tiles2 * Hkv >= kTargetGroups ? 2 : 1;
+// A kernel form of one head dim: 16-query blocks per wave, stage halves or not, and its
+// cost in us with one workgroup per CU: `wg` per workgroup (Q and first-stage loads, the
+// pipeline's fill, epilogue) and `stage` per 32-key stage.  Fitted to graph-replayed times
+// over 1 .. 470 stages and 4 .. 512 workgroups; the plans then lie within 5% of the best
+// forced split on 40 of 45 random chunks (the others within 14%).
+struct Tiling {
+    int qb, kh;
+    float wg, stage;
+    int rows() const { return 16 * qb * (kh ? kWaves / 2 : kWaves); }
+};
+
+// The forms a head dim can run.  At D = 256, per 32 keys: 64-row stage-halves tiles 0.66 us,
+// 128-row tiles 1.16, and 256-row tiles, whose two blocks share each K and V read, 1.9.
+constexpr Tiling kTilings512[] = {{1, 0, 9.0f, 1.5f}};
+constexpr Tiling kTilings256[] = {{1, 1, 5.5f, 0.66f}, {1, 0, 5.5f, 1.16f}, {2, 0, 8.0f, 1.9f}};
+constexpr Tiling kTilings128[] = {{2, 0, 3.5f, 1.0f}};
+
+// Estimated us of a plan: `pieces(f)` calls f(stages) for each workgroup of one kv head in
+// dispatch order.  The heads run side by side, so one head has kTargetGroups / Hkv CUs; the
+// dispatcher hands a workgroup to the CU that falls idle first, which for the descending
+// lengths of the tiles (latest first) is the order back and forth over the CUs.
+template <class F>
+float makespan(int Hkv, const Tiling &t, F &&pieces) {
+    const int cus = std::max(1, kTargetGroups / Hkv);
+    const float share = Hkv > kTargetGroups ? (float) Hkv / kTargetGroups : 1.0f;  // heads per CU
+    float load[kTargetGroups];
+    std::fill_n(load, cus, 0.0f);
+    int at = 0, dir = 1;
+    pieces([&](int stages) {
+        load[at] += t.wg + stages * t.stage;
+        if (at + dir < 0 || at + dir >= cus) dir = -dir;  // the end takes two in a row
+        else at += dir;
+    });
+    float most = 0.0f;
+    for (int i = 0; i < cus; ++i) most = std::max(most, load[i]);
+    return most * share;
 }
 
-// Stage halves (the KH kernel, 64-row tiles) at D = 256 with one block per wave, when the
-// 128-row tiles alone would leave CUs idle: twice the tiles instead of key splits.
-bool pick_kh(int D, int qb, long long rows, int Hkv) {
-    if (D != 256 || qb != 1) return false;
-    const long long tiles1 = (rows + 16 * kWaves - 1) / (16 * kWaves);
-    return tiles1 * Hkv < kTargetGroups;
-}
+// Splitting adds a dependent launch (us) and D fp32 per row and split, written by the
+// attention kernel and read by the merge (us per byte).
+constexpr float kSplitLaunch = 6.5f, kPartialByte = 3.1e-7f;
+constexpr int kMaxRounds = 3;  // split plans of more workgroups per CU only add partials
 
 // Validates a description and fills the kernel parameters' shape fields and plan.
 int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
@@ -819,34 +844,67 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
     p->o_rs = d->out_row_stride;
     p->o_hs = d->out_head_stride;
     p->scale_log2e = d->scale * 1.4426950408889634f;
-    p->qb = pick_qb(D, (long long) d->seq_q * p->G, d->num_kv_heads);
-    p->kh = pick_kh(D, p->qb, (long long) d->seq_q * p->G, d->num_kv_heads) ? 1 : 0;
-    const int QT = 16 * p->qb * (p->kh ? kWaves / 2 : kWaves);
-    const long long tiles = ((long long) d->seq_q * p->G + QT - 1) / QT;
-    if (tiles * d->num_kv_heads > (1LL << 24))
-        return fail(ESDA_ERR_INVALID_ARGUMENT, "esda_prefill: too many query tiles");
-    p->tiles = (int) tiles;
-    // The widest key range of any tile (the last one under a causal mask).
-    int maxn = 0;
-    for (int t = 0; t < p->tiles; ++t) {
-        int a, b;
-        tile_keys(*p, t, QT, a, b);
-        maxn = std::max(maxn, b - a);
+    // Form and split: the cheapest by the cost above.  What counts is how the workgroups fill
+    // rounds of 256 CUs: 333 queries over 5933 keys (84 tiles) take 135 us as 252 workgroups
+    // and 192 us as 336, whose second round is mostly idle; 770 fresh tokens (192 tiles) 51 us
+    // unsplit and 80 us split in two.
+    const long long rows = (long long) d->seq_q * p->G;
+    const Tiling *forms = D == 512 ? kTilings512 : D == 256 ? kTilings256 : kTilings128;
+    const int nforms = D == 256 ? 3 : 1;
+    float best = INFINITY;
+    int kps = 0, most_stages = 0;  // of the best plan
+    for (int f = 0; f < nforms; ++f) {
+        const Tiling &t = forms[f];
+        const int QT = t.rows();
+        const long long tiles = (rows + QT - 1) / QT, groups = tiles * d->num_kv_heads;
+        if (groups > (1LL << 24)) {
+            if (f + 1 < nforms) continue;
+            return fail(ESDA_ERR_INVALID_ARGUMENT, "esda_prefill: too many query tiles");
+        }
+        const bool few = groups <= kMaxRounds * kTargetGroups;
+        int nst[kMaxRounds * kTargetGroups];  // few: stages of each tile, latest first
+        int most = 1;
+        double total = 0.0;
+        for (int i = 0; i < (int) tiles; ++i) {
+            int a, b;
+            tile_keys(*p, (int) tiles - 1 - i, QT, a, b);
+            const int n = (b - a + kStageKeys - 1) / kStageKeys;
+            if (few) nst[i] = n;
+            most = std::max(most, n);
+            total += t.wg + n * t.stage;
+        }
+        auto consider = [&](int per) {  // per: stages per split
+            const int splits = (most + per - 1) / per;
+            float us = splits > 1 ? kSplitLaunch + kPartialByte * 4.0f * D * (float) rows * d->num_kv_heads * splits : 0.0f;
+            if (us + t.wg + per * t.stage >= best) return splits;
+            if (few)
+                us += makespan(d->num_kv_heads, t, [&](auto &&piece) {
+                    for (int i = 0; i < (int) tiles; ++i)
+                        for (int j = 0; j < nst[i]; j += per) piece(std::min(per, nst[i] - j));
+                });
+            else  // many rounds: the CUs stay busy but for the end of the last
+                us += (float) (total * d->num_kv_heads / kTargetGroups) + 0.5f * (t.wg + most * t.stage);
+            if (us < best) {
+                best = us;
+                kps = per * kStageKeys;
+                most_stages = most;
+                p->qb = t.qb;
+                p->kh = t.kh;
+                p->tiles = (int) tiles;
+            }
+            return splits;
+        };
+        if (d->split_keys > 0) {
+            consider(few ? d->split_keys / kStageKeys : most);
+        } else {
+            consider(most);
+            for (int s = 2; s <= most && groups * s <= kMaxRounds * kTargetGroups;)
+                s = std::max(s, consider((most + s - 1) / s)) + std::max(1, s / 4);
+        }
     }
-    int kps;
-    if (d->split_keys > 0) {
-        kps = d->split_keys;
-    } else {
-        // enough workgroups to cover the CUs, each with at least 8 stages
-        const long long groups = tiles * d->num_kv_heads;
-        long long s = (kTargetGroups + groups - 1) / groups;
-        const long long smax = std::max<long long>(1, maxn / (8 * kStageKeys));
-        s = std::min(s, smax);
-        kps = (int) (((maxn + s - 1) / s + kStageKeys - 1) / kStageKeys * kStageKeys);
-    }
-    if (kps <= 0) kps = kStageKeys;
-    const long long splits = (maxn + kps - 1) / kps;
-    if (splits > 65535 || tiles * d->num_kv_heads * splits > INT_MAX)
+    if (d->split_keys > 0) kps = d->split_keys;
+    const long long splits = ((long long) most_stages * kStageKeys + kps - 1) / kps;
+    if (splits > 65535 || (long long) p->tiles * d->num_kv_heads * splits > INT_MAX)
         return fail(ESDA_ERR_INVALID_ARGUMENT, "esda_prefill: too many key splits");
     p->kps = kps;
     p->splits = (int) std::max<long long>(1, splits);

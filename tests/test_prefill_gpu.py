@@ -127,6 +127,38 @@ def test_global_chunk_after_cached_past_auto_splits():
     run_prefill("global-chunk", Hq=32, Hkv=4, D=512, Sq=64, Sk=1000, q_pos0=936, k_pos0=0, seed=2)
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,Sq,Sk,split_keys", [
+    (512, 8, 1, 9, 2120, 32),     # 67 splits: more than a wave's lanes, the last one short
+    (256, 6, 3, 50, 900, 64),     # 15 splits, the early rows see fewer of them
+    (128, 4, 4, 70, 70, 32),      # fresh: splits past a row's position are empty
+    (512, 2, 2, 1, 289, 32),      # one row, a last split of one key
+])
+def test_split_merge_counts(D, Hq, Hkv, Sq, Sk, split_keys):
+    """The split merge over more splits than lanes, counts that leave a short batch of rows
+    in flight, and rows whose later splits hold no key."""
+    run_prefill(f"merge-{D}", Hq=Hq, Hkv=Hkv, D=D, Sq=Sq, Sk=Sk, q_pos0=Sk - Sq, k_pos0=0, split_keys=split_keys,
+                seed=31 + D)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,Sq,past,window", [
+    (512, 32, 4, 257, 700, 0),     # 17 tiles a head, the last of 8 rows: three splits fill one round
+    (512, 16, 2, 16, 4900, 0),     # one full tile a head: tens of splits
+    (512, 8, 8, 129, 0, 0),        # fresh, a last tile of one row
+    (256, 32, 16, 1100, 0, 256),   # 128-row tiles just past one round of the CUs
+    (256, 16, 8, 17, 2000, 1024),  # short chunk: stage halves and splits together
+    (256, 16, 8, 2470, 0, 1024),   # 128-row tiles in two uneven rounds
+    (256, 32, 16, 4001, 1341, 1024),  # 256-row tiles, stages off the grid, a short last tile
+    (128, 8, 4, 300, 1500, 0),     # 256-row tiles with splits
+])
+def test_planned_forms_and_splits(D, Hq, Hkv, Sq, past, window):
+    """Automatic plans at the edges of the form and split choice: sampled rows (the first and
+    last of the chunk, of its tiles and of the tiles' ragged end)."""
+    Sk = min(past + Sq, window + Sq) if window else past + Sq
+    rows = sorted({0, 1, 15, 16, 31, 32, 63, 64, 127, 128, 255, 256, Sq // 2, Sq - 2, Sq - 1} & set(range(Sq)))
+    run_prefill(f"plan-{D}-{Sq}", Hq=Hq, Hkv=Hkv, D=D, Sq=Sq, Sk=Sk, q_pos0=past, k_pos0=past + Sq - Sk,
+                window=window, seed=51, rows=rows, shared=D == 512 and Hkv == 4)
+
+
 def test_local_sliding_window_with_evicted_keys():
     # chunked prefill keeps window + seq keys (ESAttention.mm:99-103): pastLen 500
     run_prefill("local-window", Hq=8, Hkv=4, D=256, Sq=200, Sk=264, q_pos0=500, k_pos0=436, window=64, seed=3)
