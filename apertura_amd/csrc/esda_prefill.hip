@@ -570,25 +570,65 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
 }
 
 // out(i, h, :) = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the splits with
-// l_s > 0.  One wave per (row, 64 * VEC dims): lane j first loads (m, l) of split j (and
-// j + 64, ..), so the max, the weights and the denominator take one round trip and wave
-// reductions; the wave then walks the live splits (a ballot: wave-uniform, so an empty
-// split costs nothing) with MB of their partial rows in flight.
-// Memory-bound: splits * D * 4 bytes per row, read once.  A thread per 4 dims walking the
-// splits one after another was bound by their latency instead: 512 rows of D = 512 with 18
-// splits 8.2 us against 4.3 here, with 32 splits 19.9 against 6.3.
-template <int D>
+// l_s > 0.  One wave per (row, 64 * VEC dims).  Memory-bound: splits * D * 4 bytes per row,
+// read once, so the two forms differ in how they cover the latency:
+//  - NS > 0, for plans of at most NS splits: every (m, l) and partial row is loaded at once
+//    (one round trip; a row that an empty split never wrote is dropped by a select);
+//  - NS = 0: lane j loads (m, l) of split j (and j + 64, ..), so the max, the weights and the
+//    denominator take one round trip and wave reductions, and the wave then walks the live
+//    splits (a ballot: wave-uniform) with MB of their rows in flight.
+// A thread per 4 dims walking the splits one after another was bound by their latency:
+// 512 rows of D = 512 with 18 splits 8.2 us against 4.3 here, with 32 splits 19.9 against
+// 6.3; 16384 rows with 2 splits 17.2 against 14.4 (67 MB at 4.7 TB/s).
+template <int D, int NS>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     constexpr int VEC = D >= 256 ? 4 : D / 64;  // dims per lane
     constexpr int PARTS = D / (64 * VEC);       // waves per row
     constexpr int MB = 8;                       // partial rows in flight
     typedef float vec __attribute__((ext_vector_type(VEC)));
+    typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
     const int lane = threadIdx.x & 63;
     const long long nrows = (long long) p.Sq * p.Hq;
     const long long wv = (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
     if (wv >= nrows * PARTS) return;
     const long long row = wv / PARTS;
     const int d0 = (int) (wv % PARTS) * 64 * VEC + lane * VEC;
+    const float *acc = p.part_acc + row * D + d0;
+    const long long ss = nrows * D;
+    auto write = [&](const vec &v) {
+        bvec b;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) b[e] = (__bf16) v[e];
+        const int i = (int) (row / p.Hq), h = (int) (row % p.Hq);
+        *reinterpret_cast<bvec *>(p.out + (size_t) i * p.o_rs + (size_t) h * p.o_hs + d0) = b;
+    };
+    if constexpr (NS > 0) {
+        f32x2 mls[NS];
+        vec a[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            mls[s] = f32x2{-INFINITY, 0.0f};
+            a[s] = 0.0f;
+            if (s < p.splits) {
+                mls[s] = *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row));
+                a[s] = *reinterpret_cast<const vec *>(acc + s * ss);
+            }
+        }
+        float M = -INFINITY, den = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) M = mls[s][1] > 0.0f ? fmaxf(M, mls[s][0]) : M;
+        vec num = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const bool live = mls[s][1] > 0.0f;
+            const float w = live ? __builtin_amdgcn_exp2f(mls[s][0] - M) : 0.0f;
+            den += live ? mls[s][1] * w : 0.0f;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) num[e] += live ? w * a[s][e] : 0.0f;
+        }
+        write(num * (1.0f / den));
+        return;
+    }
     auto ml_of = [&](int s) {
         return s < p.splits ? *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row))
                             : f32x2{-INFINITY, 0.0f};
@@ -603,8 +643,6 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
     float den = 0.0f;
     vec num = 0.0f;
-    const float *acc = p.part_acc + row * D + d0;
-    const long long ss = nrows * D;
     for (int s0 = 0; s0 < p.splits; s0 += 64) {
         if (s0) ml = ml_of(s0 + lane);
         const float w = ml[1] > 0.0f ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.0f;
@@ -630,13 +668,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) den += __shfl_xor(den, o);
-    const vec v = num * (1.0f / den);
-    typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
-    bvec b;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) b[e] = (__bf16) v[e];
-    const int i = (int) (row / p.Hq), h = (int) (row % p.Hq);
-    *reinterpret_cast<bvec *>(p.out + (size_t) i * p.o_rs + (size_t) h * p.o_hs + d0) = b;
+    write(num * (1.0f / den));
 }
 
 // ------------------------------------------------------------ raw-K reconstruction
@@ -936,7 +968,10 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
     }
     if ((stages & 2) && p.splits > 1) {
         const long long waves = (long long) p.Sq * p.Hq * (D >= 256 ? D / 256 : 1);
-        hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st, p);
+        const dim3 grid((unsigned) ((waves + 3) / 4)), block(256);
+        if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, p);
+        else if (p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((prefill_merge_kernel<D, 0>), grid, block, 0, st, p);
     }
 }
 
