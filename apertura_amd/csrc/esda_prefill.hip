@@ -673,9 +673,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 
 // ------------------------------------------------------------ raw-K reconstruction
 //
-// One wave per key row.  Lane l holds dims HP*l .. +HP of each half (HP = D/128), so each
-// rotary pair (d, d + D/2) sits in one lane.  The sum of squares is an fp32 wave
-// reduction; rinv = 1 / sqrt(mean + eps) with IEEE division and square root.
+// Memory-bound: a raw row read, a K and a V row written.  LPR = D/16 lanes hold a row, each
+// 8 dims of either half (16-byte loads and stores; every rotary pair (d, d + D/2) in one
+// lane), so a wave holds 64/LPR consecutive rows, and it does HG kv heads of them: their
+// loads are in flight together and share one set of cos / sin and k-norm weights.  4 heads
+// x 8256 rows 20.0 us (5.1 TB/s), x 16384 rows 33.5 (6.0); one wave per row with 8-byte
+// accesses, its own cos / sin and its own weight loads took 33.1 and 58.1.  The sum of squares is an fp32 sum over the row's lanes; rinv =
+// 1 / sqrt(mean + eps) with IEEE division and square root.
 struct RawKvParams {
     const uint16_t *raw;        // bf16 rows, or NULL with q8 / scale / bias
     const unsigned char *q8;
@@ -690,51 +694,94 @@ struct RawKvParams {
 
 __device__ __forceinline__ float bf16r(float x) { return (float) (__bf16) x; }
 
-template <int D, bool Q8>
+// Callers' rows need only their element's alignment.
+typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned u32x2_a1 __attribute__((ext_vector_type(2), aligned(1)));
+
+template <int D, bool Q8, int HG>
 __global__ __launch_bounds__(256) void raw_prefill_kv_kernel(RawKvParams p) {
 #pragma clang fp contract(off)  // every rounding point as written (no fused multiply-add)
-    constexpr int HP = D / 128, HALF = D / 2;
-    const int lane = threadIdx.x & 63;
-    const long long gw = (long long) blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (gw >= (long long) p.Hkv * p.rows) return;
-    const int h = (int) (gw / p.rows), t = (int) (gw % p.rows);
-    float x[2][HP];
+    constexpr int HALF = D / 2, LPR = D / 16, RPW = 64 / LPR;
+    const int lane = threadIdx.x & 63, l = lane % LPR;
+    const long long wv = (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+    const int row_groups = (p.rows + RPW - 1) / RPW;
+    const int h0 = (int) (wv / row_groups) * HG;
+    if (h0 >= p.Hkv) return;
+    const int tt = (int) (wv % row_groups) * RPW + lane / LPR;
+    const int t = min(tt, p.rows - 1);  // rows past the end repeat the last one, unwritten
+
+    u32x4 raw[HG][2];
+    float sc[HG], bs[HG];
 #pragma unroll
-    for (int half = 0; half < 2; ++half)
+    for (int g = 0; g < HG; ++g) {
+        const int h = min(h0 + g, p.Hkv - 1);
 #pragma unroll
-        for (int e = 0; e < HP; ++e) {
-            const int d = half * HALF + HP * lane + e;
+        for (int half = 0; half < 2; ++half) {
+            const size_t at = (size_t) h * p.raw_hs + (size_t) t * D + half * HALF + 8 * l;
             if constexpr (Q8) {
-                const size_t r = (size_t) h * p.sb_hs + t;
-                const float prod = (float) p.q8[(size_t) h * p.raw_hs + (size_t) t * D + d] * p.sc[r];
-                x[half][e] = bf16r(prod + p.bs[r]);  // the bf16 raw view of the q8 row
+                const u32x2 w = *reinterpret_cast<const u32x2_a1 *>(p.q8 + at);
+                raw[g][half] = u32x4{w[0], w[1], 0u, 0u};
             } else {
-                x[half][e] = __builtin_bit_cast(float, (unsigned) p.raw[(size_t) h * p.raw_hs + (size_t) t * D + d] << 16);
+                raw[g][half] = *reinterpret_cast<const u32x4_a2 *>(p.raw + at);
             }
         }
-    float ss = 0.0f;
-#pragma unroll
-    for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int e = 0; e < HP; ++e) ss += x[half][e] * x[half][e];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
-    const float rinv = 1.0f / sqrtf(ss / (float) D + p.eps);
-    uint16_t *ko = p.k + (size_t) h * p.out_hs + (size_t) t * D;
-    uint16_t *vo = p.v + (size_t) h * p.out_hs + (size_t) t * D;
+        if constexpr (Q8) {
+            sc[g] = p.sc[(size_t) h * p.sb_hs + t];
+            bs[g] = p.bs[(size_t) h * p.sb_hs + t];
+        }
+    }
+    const u32x4 kwa = *reinterpret_cast<const u32x4_a2 *>(p.kw + 8 * l);
+    const u32x4 kwb = *reinterpret_cast<const u32x4_a2 *>(p.kw + HALF + 8 * l);
+    auto bf = [](const u32x4 &w, int e) { return e & 1 ? bf16_hi(w[e / 2]) : bf16_lo(w[e / 2]); };
+    float c[8], s[8];
     const float pos = (float) (p.pos0 + t);
 #pragma unroll
-    for (int e = 0; e < HP; ++e) {
-        const int d = HP * lane + e;
-        const float k0a = bf16r(x[0][e] * rinv * __builtin_bit_cast(float, (unsigned) p.kw[d] << 16));
-        const float k0b = bf16r(x[1][e] * rinv * __builtin_bit_cast(float, (unsigned) p.kw[d + HALF] << 16));
+    for (int e = 0; e < 8; ++e) {
         float sn, cs;
-        sincos_f32(pos * p.inv_freq[d], sn, cs);
-        const float c = bf16r(cs), s = bf16r(sn);
-        ko[d] = __builtin_bit_cast(uint16_t, (__bf16) (bf16r(k0a * c) + bf16r(-k0b * s)));
-        ko[d + HALF] = __builtin_bit_cast(uint16_t, (__bf16) (bf16r(k0b * c) + bf16r(k0a * s)));
-        vo[d] = __builtin_bit_cast(uint16_t, (__bf16) (x[0][e] * rinv));
-        vo[d + HALF] = __builtin_bit_cast(uint16_t, (__bf16) (x[1][e] * rinv));
+        sincos_f32(pos * p.inv_freq[8 * l + e], sn, cs);
+        c[e] = bf16r(cs);
+        s[e] = bf16r(sn);
+    }
+#pragma unroll
+    for (int g = 0; g < HG; ++g) {
+        if (h0 + g >= p.Hkv) break;
+        float x[2][8];
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if constexpr (Q8) {
+                    const float prod = (float) ((raw[g][half][e / 4] >> (8 * (e % 4))) & 255u) * sc[g];
+                    x[half][e] = bf16r(prod + bs[g]);  // the bf16 raw view of the q8 row
+                } else {
+                    x[half][e] = bf(raw[g][half], e);
+                }
+            }
+        float ss = 0.0f;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[half][e] * x[half][e];
+#pragma unroll
+        for (int o = LPR / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+        const float rinv = 1.0f / sqrtf(ss / (float) D + p.eps);
+        bf16x8 ka, kb, va, vb;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float k0a = bf16r(x[0][e] * rinv * bf(kwa, e));
+            const float k0b = bf16r(x[1][e] * rinv * bf(kwb, e));
+            ka[e] = (__bf16) (bf16r(k0a * c[e]) + bf16r(-k0b * s[e]));
+            kb[e] = (__bf16) (bf16r(k0b * c[e]) + bf16r(k0a * s[e]));
+            va[e] = (__bf16) (x[0][e] * rinv);
+            vb[e] = (__bf16) (x[1][e] * rinv);
+        }
+        if (tt < p.rows) {
+            const size_t at = (size_t) (h0 + g) * p.out_hs + (size_t) t * D + 8 * l;
+            *reinterpret_cast<u32x4_a2 *>(p.k + at) = __builtin_bit_cast(u32x4, ka);
+            *reinterpret_cast<u32x4_a2 *>(p.k + at + HALF) = __builtin_bit_cast(u32x4, kb);
+            *reinterpret_cast<u32x4_a2 *>(p.v + at) = __builtin_bit_cast(u32x4, va);
+            *reinterpret_cast<u32x4_a2 *>(p.v + at + HALF) = __builtin_bit_cast(u32x4, vb);
+        }
     }
 }
 
@@ -975,21 +1022,29 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
     }
 }
 
+constexpr long long kRawKvWaves = 4 * kTargetGroups;
+
+template <int D, bool Q8>
+void launch_raw_kv(const RawKvParams &p, hipStream_t st) {
+    // Two heads per wave once that leaves a wave for every SIMD, else one: short chunks are
+    // bound by the latency of one wave's work (4 heads x 512 rows 4.2 us with one, 4.7 with
+    // two; x 3000 rows 9.4 with two, 10.3 with four).
+    const long long groups = (p.rows + (1024 / D) - 1) / (1024 / D);  // 64 / (D / 16) rows each
+    const bool wide = groups * ((p.Hkv + 1) / 2) >= kRawKvWaves;
+    const long long waves = groups * (wide ? (p.Hkv + 1) / 2 : p.Hkv);
+    const dim3 grid((unsigned) ((waves + 3) / 4)), block(256);
+    if (wide) hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 2>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 1>), grid, block, 0, st, p);
+}
+
 int run_raw_kv(const RawKvParams &p, int D, bool q8, hipStream_t st) {
     int rc = esda_detail::check_device();
     if (rc != ESDA_OK) return rc;
-    const long long waves = (long long) p.Hkv * p.rows;
-    if (waves == 0) return ESDA_OK;
-    const dim3 grid((unsigned) ((waves + 3) / 4)), block(256);
-    if (q8) {
-        hipLaunchKernelGGL((raw_prefill_kv_kernel<512, true>), grid, block, 0, st, p);
-    } else if (D == 512) {
-        hipLaunchKernelGGL((raw_prefill_kv_kernel<512, false>), grid, block, 0, st, p);
-    } else if (D == 256) {
-        hipLaunchKernelGGL((raw_prefill_kv_kernel<256, false>), grid, block, 0, st, p);
-    } else {
-        hipLaunchKernelGGL((raw_prefill_kv_kernel<128, false>), grid, block, 0, st, p);
-    }
+    if (p.rows == 0) return ESDA_OK;
+    if (q8) launch_raw_kv<512, true>(p, st);
+    else if (D == 512) launch_raw_kv<512, false>(p, st);
+    else if (D == 256) launch_raw_kv<256, false>(p, st);
+    else launch_raw_kv<128, false>(p, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(ESDA_ERR_HIP, std::string("raw_prefill_kv launch: ") + hipGetErrorString(e));
     return ESDA_OK;

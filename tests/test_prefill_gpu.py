@@ -368,6 +368,35 @@ def test_raw_q8_prefill_kv_matches_the_oracle():
     _close_bf16(_host(v), ev, "q8 V")
 
 
+@pytest.mark.parametrize("D,Hkv,rows,q8", [(512, 3, 1025, False), (256, 5, 1403, False), (128, 3, 4099, False),
+                                           (512, 3, 1027, True), (512, 1, 1, False)])
+def test_raw_prefill_kv_many_rows(D, Hkv, rows, q8):
+    """Enough rows that a wave takes two kv heads, with an odd head and rows that end inside
+    a wave; inputs and weights at odd element offsets (rows need only element alignment)."""
+    from apertura_amd.prefill import raw_prefill_kv, raw_q8_prefill_kv
+    rng = np.random.default_rng(60 + D + q8)
+    raw, kw = _raw_inputs(rng, Hkv, rows, D)
+    inv = orc.rope_inv_freq(D, 1.0e6, 0.25)
+
+    def odd(t):  # the same rows one element past an allocation's start
+        b = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        b[1:] = t.reshape(-1).cuda()
+        return b[1:].view(t.shape)
+
+    kwd, invd = odd(_dev(kw)), odd(torch.from_numpy(inv))
+    if q8:
+        qc, sc, bs = orc.quantize_rows(raw)
+        k, v = raw_q8_prefill_kv(odd(torch.from_numpy(qc)), torch.from_numpy(sc).cuda(), torch.from_numpy(bs).cuda(),
+                                 kwd, 1e-6, invd, 7)
+        raw = orc.to_bf16((qc.astype(np.float32) * sc[..., None]).astype(np.float32) + bs[..., None])
+    else:
+        k, v = raw_prefill_kv(odd(_dev(raw)), kwd, 1e-6, invd, 7)
+    torch.cuda.synchronize()
+    ek, ev = orc.raw_prefill_kv(raw, kw, 1e-6, inv, 7)
+    _close_bf16(_host(k), ek, f"K d{D} rows{rows}")
+    _close_bf16(_host(v), ev, f"V d{D} rows{rows}")
+
+
 def test_raw_prefill_end_to_end():
     """ESAttention.mm:306-332: reconstruct K / V from the raw stream (keys at positions
     0 .. seqK-1), then prefill attention of the chunk at pastLen."""
