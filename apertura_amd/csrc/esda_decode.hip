@@ -9,7 +9,7 @@
 //
 // Kernels
 //   attend_kernel  grid (splits, kv heads, sequences) or balanced shares of a ragged
-//                  batch; 4 or 8 waves, one workgroup per CU (two at D = 256), the
+//                  batch; 4 waves, one workgroup per CU (two at D = 256), the
 //                  ring in the whole LDS or in half of it.  A workgroup streams
 //                  visible rows of one (sequence, kv head) -- or of 2 or 4 kv heads
 //                  packed together -- through an LDS ring filled by LDS DMA, splits the head dim across its
@@ -17,6 +17,7 @@
 //                  runs an fp32 online softmax and writes (m, l, acc) partials.  The
 //                  workgroup whose split ends at the new token also copies its row into
 //                  the cache.  Details at the kernel.
+//   raw_attend_kernel  the same over a raw-K or q8 raw-K stream, K and V rebuilt per row.
 //   merge_kernel   reduces the partials of all splits per (sequence, query head).
 //   append_kernel  multi-row append (slice_update) for prefill-style callers.
 // The C ABI (include/esda.h) is at the end of the file.
@@ -97,9 +98,8 @@ struct AttendParams {
 // 32 B pad), sub-row q at +2D*q bytes.  The 32-byte pad (a measured choice: 16 B leaves
 // both the 128-bit row reads and the transpose reads 2-way bank-conflicted on gfx950)
 // makes both read patterns conflict-free with every address a base plus an immediate.
-// EXTRA: LDS bytes the kernel variant needs beside the ring and the score exchange; PSX:
-// LDS bytes it keeps per ring stage beside the rows.
-template <int D, bool SHARED, int NW, int EXTRA = 0, int PSX = 0, int LDSB = 160 * 1024>
+// LDSB: the LDS bytes of one workgroup.
+template <int D, bool SHARED, int NW, int LDSB>
 struct Ring {
     static constexpr int RPI = 512 / D;                     // rows per DMA instruction
     static constexpr int NI = 16 / RPI;                     // DMA instructions per stage
@@ -116,7 +116,7 @@ struct Ring {
     static constexpr int XB = 2 * NW * 64 * 16;             // score-exchange bytes
     // reserve: kernel arguments' spill room (256 B) and the batch prefix scan (int64 per
     // sequence + one per wave)
-    static constexpr int NS_ = (LDSB - XB - 256 - ((kMaxBatch + 1) + NW) * 8 - EXTRA) / (SB + PSX);
+    static constexpr int NS_ = (LDSB - XB - 256 - ((kMaxBatch + 1) + NW) * 8) / SB;
     static constexpr int NS = NS_ > 16 ? 16 : NS_;          // stages in the ring
     static_assert(DW % 32 == 0 && NI % NW == 0, "wave slices must cover whole MFMA steps");
     static_assert(NS >= 4, "the ring needs at least 4 stages");
@@ -137,24 +137,6 @@ struct Ring {
 
 constexpr int kRawDim = 512;
 constexpr int kRopePairs = 64;
-constexpr int kTabStride = 68;  // words per cos/sin table row: 64 + 4 (conflict-free 128-bit reads)
-// LDS of the raw-mode exchanges for NW waves, in this order: row sums of squares
-// [3][16][NW], the row factors [2][3][16], (q8) the row sums [3][16][NW], and the cos/sin
-// tables [2][16][kTabStride] computed in the kernel.
-constexpr int raw_extra_lds(int nw, bool q8 = false) {
-    return 3 * 16 * nw * 4 + 2 * 3 * 16 * 4 + (q8 ? 3 * 16 * nw * 4 : 0) + 2 * 16 * kTabStride * 4;
-}
-// q8 raw-K mode: u8 stages are widened into bf16 staging slots laid out as the D = 512
-// ring (16 rows of 1056-byte blocks), four deep; per-row scale / bias ride beside each
-// u8 stage.
-constexpr int kQ8Stage = 16 * 1056;
-constexpr int kQ8Slots = 4;
-constexpr int kQ8SbStages = 16;
-constexpr int q8_extra_lds(int nw) {
-    return raw_extra_lds(nw, true) + kQ8Slots * kQ8Stage + kQ8SbStages * 2 * 16 * 4;
-}
-
-
 // The segments of one launch's workgroup: grid plans give workgroup (split, kv head,
 // sequence) rows [split * chunk, ...) of its pair; balanced plans give workgroup w its share
 // of all visible rows of the batch, walked pair by pair (esda_plan.h).  segment(b, kvh, j0,
@@ -294,7 +276,7 @@ __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segme
 
 // --------------------------------------------------------------------- attend kernel
 //
-// grid (splits, kv heads, sequences), NW = 4 or 8 waves per workgroup, the ring in 1/OCC of
+// grid (splits, kv heads, sequences), NW waves per workgroup, the ring in 1/OCC of
 // the LDS (so that OCC workgroups fit per CU).  A workgroup owns `chunk` consecutive visible rows
 // of one (sequence, kv head) and streams them through the LDS ring in 16-row stages.
 // When each pair needs one split and pairs are plentiful, pk = 2 or 4 kv heads of a
@@ -312,49 +294,27 @@ __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segme
 // transpose reads).  One barrier per stage: the scores of stage s+1 are formed while
 // stage s is accumulated.  With attention_k_eq_v the V rows are the K rows in LDS.
 //
-// RAW (D = 512, one tensor): the QK operand is rebuilt from raw rows in registers.  The
-// row norms need all four waves' dims, so each stage's partial sums of squares (and its
-// cos/sin table) are published two stages ahead: in iteration s the waves publish
-// stage s+2's sums and table, form stage s+1's scores and accumulate stage s.
-//
 // The new token's row is copied from k_new/v_new into the cache by the workgroup whose
 // split ends at it (bit-exact copy); that workgroup's own loads read the row from
 // k_new/v_new and no other workgroup reads it, so the copy needs no ordering.
-//
-// Q8 (raw mode over a q8 raw stream, esDecodeAttnGlobalQ8, ESDecodeAttn.mm:275-369): rows
-// are u8 with a per-row scale and bias, x = q * scale + bias.  The u8 ring (512-byte rows)
-// is widened into bf16 staging slots three stages ahead, where q is exact, so the raw
-// pipeline runs on q itself: the Gram diagonal and a row sum give sum(q^2) and sum(q)
-// exactly, hence sum(x^2); K = bf16(rope(fma(q, scale*rinv, bias*rinv) * kw)); V enters
-// as q with the weight P = bf16(e * scale * rinv) and the bias as sum P * bias / scale.
-// The workgroup holding a sequence's new row quantizes it into the cache first.
-template <int D, bool SHARED, int NW, bool RAW, bool Q8 = false, int OCC = 1>
+template <int D, bool SHARED, int NW, int OCC = 1>
 // The LDS ring allows OCC workgroups per CU, i.e. OCC * NW/4 waves per SIMD: telling the
 // compiler so lifts the register limit it would otherwise keep for higher occupancy,
 // which it meets by serialising LDS reads behind their uses.  (Plans may still place one
 // workgroup per CU on a kernel built with OCC = 2: its shallower ring is what they want.)
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(OCC * NW / 4, OCC * NW / 4)))
 void attend_kernel(AttendParams p) {
-    static_assert(!RAW || (D == kRawDim && SHARED && (NW == 4 || NW == 8)), "raw mode: one 512-dim stream, 4 or 8 waves");
-    static_assert(!Q8 || (RAW && NW == 8), "q8 mode is raw mode with 8 waves");
-    // R: the compute layout of a stage (and, outside q8 mode, the DMA ring); RD: the DMA ring.
-    using R = Ring<D, SHARED, NW, RAW && !Q8 ? raw_extra_lds(NW) : 0, 0, 160 * 1024 / OCC>;
-    using RD = std::conditional_t<Q8, Ring<256, true, NW, q8_extra_lds(NW)>, R>;
-    static_assert(OCC == 1 || !RAW, "raw mode holds one workgroup per CU");
+    using R = Ring<D, SHARED, NW, 160 * 1024 / OCC>;
     // D = 512 exchanges only the live heads' partial scores (the padding columns are zero)
-    constexpr bool kLiveX = D == 512 && !RAW;
-    constexpr int NS = RD::NS, DW = R::DW, KKW = R::KKW, DTW = R::DTW;
-    // DMA instructions per wave per stage (q8: the u8 rows plus one scale / bias piece)
-    constexpr int DPW = Q8 ? RD::DPT + 1 : RD::DPW;
-    // Stages between the one being accumulated and the newest one that must have landed.
-    constexpr int AHEAD = Q8 ? 3 : RAW ? 2 : 1;
-    static_assert(NS >= AHEAD + 3, "the ring must hold the look-ahead stages and one in flight");
-    static_assert(!Q8 || NS <= kQ8SbStages, "one scale / bias area per ring stage");
+    constexpr bool kLiveX = D == 512;
+    constexpr int NS = R::NS, DW = R::DW, KKW = R::KKW, DTW = R::DTW;
+    constexpr int DPW = R::DPW;  // DMA instructions per wave per stage
+    static_assert(NS >= 4, "the ring must hold the look-ahead stage and one in flight");
     // Distinct arrays per stage: the compiler tracks DMA completion per LDS object, so a
     // read of stage u only waits for stage u's DMA, never for the stages behind it.
-    __shared__ __attribute__((aligned(16))) unsigned char r0[RD::SB], r1[RD::SB], r2[RD::SB], r3[RD::SB],
-        r4[RD::SB], r5[RD::SB], r6[RD::SB], r7[RD::SB], r8[RD::SB], r9[RD::SB], r10[RD::SB], r11[RD::SB],
-        r12[RD::SB], r13[RD::SB], r14[RD::SB], r15[RD::SB];
+    __shared__ __attribute__((aligned(16))) unsigned char r0[R::SB], r1[R::SB], r2[R::SB], r3[R::SB],
+        r4[R::SB], r5[R::SB], r6[R::SB], r7[R::SB], r8[R::SB], r9[R::SB], r10[R::SB], r11[R::SB],
+        r12[R::SB], r13[R::SB], r14[R::SB], r15[R::SB];
     // Stage buffer u (a compile-time index).
     auto ring = [&](auto uc) -> unsigned char * {
         constexpr int u = decltype(uc)::value % NS;
@@ -376,28 +336,6 @@ void attend_kernel(AttendParams p) {
         else return r15;
     };
     __shared__ f32x4 xch[2][NW][64];  // partial scores, double-buffered by stage parity
-    // Raw mode: per-row partial sums of squares xss[stage % 3][row][wave], the per-row
-    // norm factors xr, and the cos/sin table xtab[stage % 2][row][pair] (bf16 cos in the low
-    // half, sin in the high half) when the kernel computes it.
-    __shared__ __attribute__((aligned(16))) unsigned char rawlds[RAW ? raw_extra_lds(NW, Q8) : 16];
-    auto *xss = reinterpret_cast<float (*)[16][NW]>(rawlds);
-    // xr[stage % 2][0][row] = the weight factor (rinv; q8: scale * rinv), [1] its inverse,
-    // [2] (q8) bias / scale
-    auto *xr = reinterpret_cast<float (*)[3][16]>(rawlds + 3 * 16 * NW * 4);
-    // q8: row sums of q [stage % 3][row][wave]
-    auto *xsq = reinterpret_cast<float (*)[16][NW]>(rawlds + 3 * 16 * NW * 4 + 2 * 3 * 16 * 4);
-    auto *xtab = reinterpret_cast<unsigned (*)[16][kTabStride]>(rawlds + 3 * 16 * NW * 4 + 2 * 3 * 16 * 4 +
-                                                                (Q8 ? 3 * 16 * NW * 4 : 0));
-    // q8: bf16 staging slots and the per-stage scale / bias rows
-    __shared__ __attribute__((aligned(16))) unsigned char q8stg[Q8 ? kQ8Slots * kQ8Stage : 16];
-    __shared__ __attribute__((aligned(16))) float q8sb[Q8 ? kQ8SbStages : 1][2][16];
-    // cos/sin table of a stage: TR rows (one per position) x 64 pairs over 64*NW threads
-    constexpr int TR = 16;
-    constexpr int EPT = TR * 64 / (64 * NW);
-    static_assert(EPT >= 1, "every thread computes at least one table entry");
-    constexpr int TPR = 64 / EPT;  // threads per table row
-
-    const int wg = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -424,15 +362,7 @@ void attend_kernel(AttendParams p) {
     uint16_t *vbase = p.v_cache + head_off;
     const uint16_t *knew = append ? p.k_new + ((size_t) b * p.Hkv + kvh) * pk * D : nullptr;
     const uint16_t *vnew = SHARED ? knew : p.v_new + ((size_t) b * p.Hkv + kvh) * pk * D;
-    // q8: the u8 rows (same element strides, in bytes) and the scale / bias rows
-    unsigned char *q8base = Q8 ? p.q8 + head_off : nullptr;
-    const size_t sb_off = Q8 ? (size_t) b * p.sb_seq_stride + (size_t) kvh * pk * p.sb_head_stride : 0;
-
-    // 32-dim chunk of the QK k-step kk of this wave.  Raw mode interleaves the waves so
-    // that each rotary pair (d, d + 256), d < 64, sits in one lane of wave 0 or 1.
-    auto qk_chunk = [&](int kk) { return RAW ? wave + NW * kk : wave * KKW + kk; };
-    // k-step holding the rotary partners (chunk + 8) of the chunk at k-step 0
-    constexpr int KP = 8 / NW;
+    auto qk_chunk = [&](int kk) { return wave * KKW + kk; };  // 32-dim chunk of QK k-step kk of this wave
 
     // Q^T operand for this wave's dims: lane (li, lg) = head li, dims 32*chunk + 8lg .. +8
     // (zero for heads >= G).
@@ -446,164 +376,53 @@ void attend_kernel(AttendParams p) {
             qv[kk] = __builtin_bit_cast(bf16x8, t);
         }
     }
-    // Raw mode: k-norm weights of the lane's QK dims, and the rotary frequencies of the
-    // four table entries this thread computes per stage (row tid/16, pairs 4(tid%16)..+4).
-    float kwf[RAW ? KKW : 1][8];
-    float invf[RAW ? EPT : 1] = {};
-    if constexpr (RAW) {
-#pragma unroll
-        for (int kk = 0; kk < KKW; ++kk) {
-            const u32x4 t = *reinterpret_cast<const u32x4 *>(p.kw + 32 * qk_chunk(kk) + 8 * lg);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                kwf[kk][2 * e] = bf16_lo(t[e]);
-                kwf[kk][2 * e + 1] = bf16_hi(t[e]);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < EPT; ++e) invf[e] = p.inv_freq[EPT * (tid % TPR) + e];
-    }
-    if constexpr (Q8) {
-        // The new row of each kv head of the group is quantized into the cache before the
-        // ring starts (wave pr: kv head pr), esQuantizeRawRows' arithmetic
-        // (ESDecodeAttn.mm:491-509): min / max over the row, scale = max((max - min) / 255,
-        // 1e-8), q = min(round((x - min) / scale), 255) rounding half away from zero, IEEE
-        // division.  The ring then reads it like every other row.
-        if (append && j1 == sv.nvis) {
-            for (int pr = wave; pr < pk; pr += NW) {
-                const u32x4 t = *reinterpret_cast<const u32x4 *>(knew + pr * D + lane * 8);
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    x[2 * e] = bf16_lo(t[e]);
-                    x[2 * e + 1] = bf16_hi(t[e]);
-                }
-                float mn = x[0], mx = x[0];
-#pragma unroll
-                for (int e = 1; e < 8; ++e) {
-                    mn = fminf(mn, x[e]);
-                    mx = fmaxf(mx, x[e]);
-                }
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    mn = fminf(mn, __shfl_xor(mn, o));
-                    mx = fmaxf(mx, __shfl_xor(mx, o));
-                }
-                float scl = (mx - mn) / 255.0f;
-                if (!(scl > 1e-8f)) scl = 1e-8f;
-                unsigned lo = 0u, hi = 0u;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const unsigned qi = (unsigned) fminf(roundf((x[e] - mn) / scl), 255.0f);
-                    if (e < 4) lo |= qi << (8 * e);
-                    else hi |= qi << (8 * (e - 4));
-                }
-                unsigned char *row = q8base + (size_t) pr * p.head_stride + (size_t) sv.newrow * kRawDim;
-                *reinterpret_cast<uint2 *>(row + lane * 8) = uint2{lo, hi};
-                if (lane == 0) {
-                    const size_t at = sb_off + (size_t) pr * p.sb_head_stride + (size_t) sv.newrow;
-                    p.qsc[at] = scl;
-                    p.qbs[at] = mn;
-                }
-            }
-        }
-    }
     ESDA_WAIT_VM(0);  // operands are in registers before the ring starts counting its own loads
-    if constexpr (Q8) lds_barrier();  // and the new row's stores are done before any wave's DMA
 
     // DMA source slot of this lane: sub-row dq, chunk dchunk of the row.
-    const int dq = lane / RD::CPR, dchunk = lane % RD::CPR;
+    const int dq = lane / R::CPR, dchunk = lane % R::CPR;
     const int nst = (j1 - j0 + RPP - 1) >> lrpp;
-    constexpr int EB = Q8 ? 1 : 2;                // bytes per cache element (strides count elements)
-    constexpr int ROWB = Q8 ? kRawDim : D * 2;    // bytes per cache row
     // Per-lane byte offsets of this wave's DMA slots inside a stage's row range (stage row
     // r: kv head r / RPP of the group, row r % RPP; below 2^31 bytes, checked by the host).
-    unsigned dvoff[RD::DPT];
+    unsigned dvoff[R::DPT];
 #pragma unroll
-    for (int t = 0; t < RD::DPT; ++t) {
-        const int r = wave * RD::DPT + t + dq * RD::NI;
-        dvoff[t] = (unsigned) ((size_t) (r >> lrpp) * p.head_stride * EB + (size_t) (r & (RPP - 1)) * ROWB + dchunk * 16);
+    for (int t = 0; t < R::DPT; ++t) {
+        const int r = wave * R::DPT + t + dq * R::NI;
+        dvoff[t] = (unsigned) ((size_t) (r >> lrpp) * p.head_stride * 2 + (size_t) (r & (RPP - 1)) * D * 2 + dchunk * 16);
     }
-    // DMA of stage st into ring buffer `buf` (ring slot `slot`).
-    auto dma = [&](int st, unsigned char *buf, int slot) {
+    // DMA of stage st into ring buffer `buf`.
+    auto dma = [&](int st, unsigned char *buf) {
         const int jst = j0 + st * RPP;
-        if constexpr (Q8) {
-            // scale / bias of the stage's rows: wave w loads the scales (w < 4) or biases of
-            // stage rows 4(w % 4) .. +3, one row per lane
-            if (lane < 4) {
-                const int sr = 4 * (wave & 3) + lane, pr = sr >> lrpp;
-                const int j = jst + (sr & (RPP - 1)), jj = j < j1 ? j : j1 - 1;
-                const float *src = (wave < 4 ? p.qsc : p.qbs) + sb_off + (size_t) pr * p.sb_head_stride +
-                                   (size_t) (sv.first + jj);
-                lds_dma4(src, lds_addr(&q8sb[slot][wave >> 2][4 * (wave & 3)]));
-            }
-        }
         if (jst + RPP < j1 && sv.first + jst + RPP <= p.cap) {
             // Interior stage: RPP consecutive cache rows per kv head, none clamped or new.
-            if constexpr (Q8) {
-                const unsigned char *qb = q8base + (size_t) (sv.first + jst) * kRawDim;
-#pragma unroll
-                for (int t = 0; t < RD::DPT; ++t) lds_dma16_s(qb, dvoff[t], lds_addr(buf) + (wave * RD::DPT + t) * RD::BLK);
-                return;
-            }
             const uint16_t *kb = kbase + (size_t) (sv.first + jst) * D;
             const uint16_t *vb = vbase + (size_t) (sv.first + jst) * D;
 #pragma unroll
-            for (int t = 0; t < RD::DPT; ++t) {
-                const int i = wave * RD::DPT + t;
-                lds_dma16_s(kb, dvoff[t], lds_addr(buf) + i * RD::BLK);
-                if constexpr (!SHARED) lds_dma16_s(vb, dvoff[t], lds_addr(buf) + RD::TB + i * RD::BLK);
+            for (int t = 0; t < R::DPT; ++t) {
+                const int i = wave * R::DPT + t;
+                lds_dma16_s(kb, dvoff[t], lds_addr(buf) + i * R::BLK);
+                if constexpr (!SHARED) lds_dma16_s(vb, dvoff[t], lds_addr(buf) + R::TB + i * R::BLK);
             }
             return;
         }
 #pragma unroll
-        for (int t = 0; t < RD::DPT; ++t) {
-            const int i = wave * RD::DPT + t;           // DMA block of this stage
-            const int sr = i + dq * RD::NI;             // stage row this lane feeds
+        for (int t = 0; t < R::DPT; ++t) {
+            const int i = wave * R::DPT + t;           // DMA block of this stage
+            const int sr = i + dq * R::NI;             // stage row this lane feeds
             const int pr = sr >> lrpp;                  // its kv head within the group
             const int j = jst + (sr & (RPP - 1));       // its logical row
             const int jj = j < j1 ? j : j1 - 1;          // clamp: masked rows read a visible row
             int r = sv.first + jj;
             if (r >= p.cap) r -= p.cap;
-            if constexpr (Q8) {
-                // the new row was quantized into the cache before the ring started
-                lds_dma16(q8base + (size_t) pr * p.head_stride + (size_t) r * kRawDim + dchunk * 16,
-                          lds_addr(buf) + i * RD::BLK);
-                continue;
-            }
             const bool from_new = append && (jj == sv.nvis - 1);
             const size_t hoff = (size_t) pr * p.head_stride + (size_t) r * D;
             const uint16_t *ks = (from_new ? knew + pr * D : kbase + hoff) + dchunk * 8;
-            lds_dma16(ks, lds_addr(buf) + i * RD::BLK);
+            lds_dma16(ks, lds_addr(buf) + i * R::BLK);
             if constexpr (!SHARED) {
                 const uint16_t *vs = (from_new ? vnew + pr * D : vbase + hoff) + dchunk * 8;
-                lds_dma16(vs, lds_addr(buf) + RD::TB + i * RD::BLK);
+                lds_dma16(vs, lds_addr(buf) + R::TB + i * R::BLK);
             }
         }
     };
-    // q8: bf16 staging slot of stage s, and the widening of u8 stage s (ring buffer u8buf)
-    // into it: thread t takes row t / 32, bytes 16 (t % 32) .. +16; a byte's bf16 is the
-    // upper half of its fp32 (exact for 0 .. 255).
-    auto stg = [&](int s) -> unsigned char * { return q8stg + (s & (kQ8Slots - 1)) * kQ8Stage; };
-    auto convert = [&](int s, const unsigned char *u8buf) {
-        if constexpr (Q8) {
-            const int r = tid >> 5, c16 = tid & 31;
-            const u32x4 w = *reinterpret_cast<const u32x4 *>(u8buf + (r & 7) * RD::BLK + (r >> 3) * kRawDim + c16 * 16);
-            unsigned o[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const unsigned lo = __builtin_bit_cast(unsigned, (float) ((w[e] >> (16 * h)) & 255u));
-                    const unsigned hi = __builtin_bit_cast(unsigned, (float) ((w[e] >> (16 * h + 8)) & 255u));
-                    o[2 * e + h] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
-                }
-            unsigned char *dst = stg(s) + r * R::BLK + c16 * 32;
-            *reinterpret_cast<u32x4 *>(dst) = u32x4{o[0], o[1], o[2], o[3]};
-            *reinterpret_cast<u32x4 *>(dst + 16) = u32x4{o[4], o[5], o[6], o[7]};
-        }
-    };
-
     // Per-lane LDS offsets: the QK A operand (row li, chunk qk_chunk(kk), 16 bytes at
     // 8lg dims) and the V^T transpose read (lane (li, lg) supplies row 4lg + li/4, dims
     // wave*DW + 16dt + 4(li%4) .. +4; ds_read_b64_tr_b16 hands lane li of the group dim
@@ -613,7 +432,6 @@ void attend_kernel(AttendParams p) {
     constexpr int VOFF = SHARED ? 0 : R::TB;
 
     float m = -INFINITY, l = 0.0f;
-    float bt = 0.0f;  // q8: sum of P * bias / scale of this lane's head (the bias part of PV)
     f32x4 acc[DTW];
 #pragma unroll
     for (int dt = 0; dt < DTW; ++dt) acc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -631,264 +449,58 @@ void attend_kernel(AttendParams p) {
         if (!kLiveX || li < p.G) xch[par][wave][lane] = sp;
     };
 
-    // ---- raw mode helpers
-    u32x4 araw[RAW ? KKW : 1];  // raw QK operand of the next stage to score
-    auto load_raw = [&](const unsigned char *kb) {
-#pragma unroll
-        for (int kk = 0; kk < (RAW ? KKW : 1); ++kk)
-            araw[kk] = *reinterpret_cast<const u32x4 *>(kb + qk_off + 64 * qk_chunk(kk));
-    };
-    // Partial sum of squares of row li over this wave's dims -> xss[buf][li][wave]: the
-    // diagonal of the stage's 16x16 Gram matrix over those dims.  The A and B operands of
-    // v_mfma_f32_16x16x32_bf16 take the same lane data (row li, dims 8lg..+8 of each
-    // chunk), and products of bf16 values are exact in the fp32 accumulation.
-    // q8: the operand is q itself, so the diagonal is sum(q^2), and an MFMA against ones
-    // gives sum(q) -> xsq; both are exact integers (per wave at most 64 * 255^2 < 2^24).
-    auto publish_ss = [&](int buf) {
-        if constexpr (RAW) {
-            f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f}, g1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            bf16x8 ones;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ones[e] = (__bf16) 1.0f;
-#pragma unroll
-            for (int kk = 0; kk < KKW; ++kk) {
-                const bf16x8 a = __builtin_bit_cast(bf16x8, araw[kk]);
-                g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, a, g, 0, 0, 0);
-                if constexpr (Q8) g1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, g1, 0, 0, 0);
-            }
-            // C layout: lane (li, lg) holds C[4lg + i][li]; row li's diagonal entry is
-            // register li - 4lg of the lanes with lg == li / 4.
-            const int i = li - 4 * lg;
-            if (i >= 0 && i < 4) {
-                xss[buf][li][wave] = i == 0 ? g[0] : i == 1 ? g[1] : i == 2 ? g[2] : g[3];
-                if constexpr (Q8) xsq[buf][li][wave] = i == 0 ? g1[0] : i == 1 ? g1[1] : i == 2 ? g1[2] : g1[3];
-            }
-        }
-    };
-    // cos/sin table of stage st: this thread's row tid / TPR, pairs EPT*(tid % TPR) .. +EPT.
-    auto publish_tab = [&](int st, int buf) {
-        if constexpr (RAW) {
-            const int row = tid / TPR;
-            const float t = (float) (sv.first + j0 + st * TR + row);
-            unsigned w[EPT];
-#pragma unroll
-            for (int e = 0; e < EPT; ++e) {
-                float s, c;
-                sincos_f32(t * invf[e], s, c);
-                w[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{c, s}, bf16x2));
-            }
-            unsigned *dst = &xtab[buf][row][EPT * (tid % TPR)];
-            static_assert(EPT == 1 || EPT == 2 || EPT == 4, "table entries per thread");
-            if constexpr (EPT == 4) {
-                *reinterpret_cast<u32x4 *>(dst) = u32x4{w[0], w[1], w[2], w[3]};
-            } else if constexpr (EPT == 2) {
-                *reinterpret_cast<uint2 *>(dst) = uint2{w[0], w[1]};
-            } else {
-                *dst = w[0];
-            }
-        }
-    };
-    // mean(kraw^2) + eps of a row; rinv = rsqrt of it.
-    auto row_ms = [&](int buf, int row) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int q4 = 0; q4 < NW; q4 += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(&xss[buf][row][q4]);
-            sum += (v[0] + v[1]) + (v[2] + v[3]);
-        }
-        return sum * (1.0f / kRawDim) + p.eps;
-    };
-    // q8: mean(x^2) + eps of a row from its sums, x = q * scale + bias: mean(x^2) =
-    // scale^2 var(q) + mean(x)^2, 512^2 var(q) = 512 sum(q^2) - sum(q)^2.  sum(q) < 2^24 is
-    // exact in fp32; sum(q^2) may round by a few units in 3.3e7, which moves var(q) by
-    // ~1e-5 of its size at most and mean(x^2) far less (the mean term carries no such error).
-    auto q8_ms = [&](int buf, int row, float scl, float bias) {
-        float s2 = 0.0f, s1 = 0.0f;
-#pragma unroll
-        for (int q4 = 0; q4 < NW; q4 += 4) {
-            const f32x4 a = *reinterpret_cast<const f32x4 *>(&xss[buf][row][q4]);
-            const f32x4 c = *reinterpret_cast<const f32x4 *>(&xsq[buf][row][q4]);
-            s2 += (a[0] + a[1]) + (a[2] + a[3]);
-            s1 += (c[0] + c[1]) + (c[2] + c[3]);
-        }
-        const float var = fmaxf(__builtin_fmaf(512.0f, s2, -s1 * s1), 0.0f);
-        const float mean = __builtin_fmaf(scl, s1 * (1.0f / kRawDim), bias);
-        return scl * scl * var * (1.0f / (kRawDim * kRawDim)) + __builtin_fmaf(mean, mean, p.eps);
-    };
-    // Scores of the stage held in araw: rebuild K in registers, then MFMA.  sbslot: the
-    // ring slot of the stage (q8: its scale / bias rows).
-    auto qk_raw = [&](int ssbuf, int tabbuf, int par, int sbslot) {
-        if constexpr (RAW) {
-            float kn[KKW][8];
-            if constexpr (Q8) {
-                const float scl = q8sb[sbslot][0][li], bias = q8sb[sbslot][1][li];
-                const float rinv = __builtin_amdgcn_rsqf(q8_ms(ssbuf, li, scl, bias));
-                const float alpha = scl * rinv, beta = bias * rinv;
-                // the weight factor scale * rinv, its inverse, and bias / scale (two IEEE
-                // divisions: written by wave 2, whose SIMD has no rotary work)
-                if (wave == 2 && lg == 0) {
-                    xr[par][0][li] = alpha;
-                    xr[par][1][li] = 1.0f / alpha;
-                    xr[par][2][li] = bias / scl;
-                }
-    #pragma unroll
-                for (int kk = 0; kk < KKW; ++kk)
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        kn[kk][2 * e] = __builtin_fmaf(bf16_lo(araw[kk][e]), alpha, beta) * kwf[kk][2 * e];
-                        kn[kk][2 * e + 1] = __builtin_fmaf(bf16_hi(araw[kk][e]), alpha, beta) * kwf[kk][2 * e + 1];
-                    }
-            } else {
-                (void) sbslot;
-                const float ms = row_ms(ssbuf, li);
-                const float rinv = __builtin_amdgcn_rsqf(ms);
-                // rinv and 1/rinv (= ms * rinv) of the row, for the stage's softmax weights.
-                if (wave == 0 && lg == 0) {
-                    xr[par][0][li] = rinv;
-                    xr[par][1][li] = ms * rinv;
-                }
-    #pragma unroll
-                for (int kk = 0; kk < KKW; ++kk)
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        kn[kk][2 * e] = bf16_lo(araw[kk][e]) * rinv * kwf[kk][2 * e];
-                        kn[kk][2 * e + 1] = bf16_hi(araw[kk][e]) * rinv * kwf[kk][2 * e + 1];
-                    }
-            }
-            if (wave < 2) {
-                // chunk `wave` (k-step 0) holds dims d = 32*wave + 8lg + e < 64; chunk wave + 8
-                // (k-step KP) their rotary partners.
-                const unsigned *tb = &xtab[tabbuf][li][32 * wave + 8 * lg];
-                const u32x4 t0 = *reinterpret_cast<const u32x4 *>(tb);
-                const u32x4 t1 = *reinterpret_cast<const u32x4 *>(tb + 4);
-    #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const unsigned w = e < 4 ? t0[e] : t1[e - 4];
-                    const float c = bf16_lo(w), s = bf16_hi(w);
-                    const float lo = kn[0][e], hi = kn[KP][e];
-                    kn[0][e] = lo * c - hi * s;
-                    kn[KP][e] = hi * c + lo * s;
-                }
-            }
-            f32x4 sp = {0.0f, 0.0f, 0.0f, 0.0f};
-    #pragma unroll
-            for (int kk = 0; kk < KKW; ++kk) {
-                bf16x8 a;
-    #pragma unroll
-                for (int e = 0; e < 8; ++e) a[e] = (__bf16) kn[kk][e];
-                sp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qv[kk], sp, 0, 0, 0);
-            }
-            xch[par][wave][lane] = sp;
-        }
-    };
-
-    // The buffer the compute reads for stage s held in ring slot uc: the ring itself, or
-    // (q8) the stage's bf16 staging slot.
-    auto cbuf = [&](int s, auto uc) -> unsigned char * {
-        if constexpr (Q8) return stg(s);
-        else return ring(uc);
-    };
-    // Prologue: fill NS-1 stages; publish what iteration 0 needs.
+    // Prologue: fill NS-1 stages; the first stage's scores.
     unroll<NS - 1>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
-        if (u < nst) dma(u, ring(uc), u);
+        if (u < nst) dma(u, ring(uc));
     });
-    if constexpr (RAW) {
-        // stages 0..2 landed (stage 2 for the first iteration's sums of squares; q8: the
-        // stages widened here)
-        if (nst - 1 >= NS - 2) {
-            ESDA_WAIT_VM((NS - 4) * DPW);
-        } else {
-            ESDA_WAIT_VM(0);
-        }
-        lds_barrier();
-        if constexpr (Q8) {
-            convert(0, ring(std::integral_constant<int, 0>{}));
-            if (nst > 1) convert(1, ring(std::integral_constant<int, 1>{}));
-            if (nst > 2) convert(2, ring(std::integral_constant<int, 2>{}));
-            lds_barrier();
-        }
-        load_raw(cbuf(0, std::integral_constant<int, 0>{}));
-        publish_ss(0);
-        publish_tab(0, 0);
-        if (nst > 1) {
-            load_raw(cbuf(1, std::integral_constant<int, 1>{}));
-            publish_ss(1);
-            publish_tab(1, 1);
-        }
-        lds_barrier();
-        // scores of stage 0 (its raw operand is read again; araw keeps stage 1's)
-        {
-            u32x4 keep[KKW];
-#pragma unroll
-            for (int kk = 0; kk < KKW; ++kk) keep[kk] = araw[kk];
-            load_raw(cbuf(0, std::integral_constant<int, 0>{}));
-            qk_raw(0, 0, 0, 0);
-#pragma unroll
-            for (int kk = 0; kk < KKW; ++kk) araw[kk] = keep[kk];
-        }
+    if (nst - 1 >= NS - 2) {
+        ESDA_WAIT_VM((NS - 2) * DPW);
     } else {
-        if (nst - 1 >= NS - 2) {
-            ESDA_WAIT_VM((NS - 2) * DPW);
-        } else {
-            ESDA_WAIT_VM(0);
-        }
-        lds_barrier();
-        qk_partial(ring(std::integral_constant<int, 0>{}), 0);
+        ESDA_WAIT_VM(0);
     }
+    lds_barrier();
+    qk_partial(ring(std::integral_constant<int, 0>{}), 0);
 
     // Iteration st: one barrier, after which (a) every wave's stage-st partial scores
-    // are in xch, (b) stage st+AHEAD has landed from every wave's DMA, and (c) every wave
+    // are in xch, (b) stage st+1 has landed from every wave's DMA, and (c) every wave
     // is done with stage st-1's buffer, which is refilled at once.  The scores of stage
     // st+1 are computed alongside stage st's PV, so the two dependency chains overlap.
     auto stage = [&](int s0, auto uc) {
         constexpr int u = decltype(uc)::value;
         const int st = s0 + u;
         if (st >= nst) return;
-        if (st + AHEAD < nst) {
-            // own DMA for stage st+AHEAD done; the stages behind it may stay in flight --
+        if (st + 1 < nst) {
+            // own DMA for stage st+1 done; the stages behind it may stay in flight --
             // except at D = 256, whose two workgroups per CU then keep twice the 512-dim
             // kernel's bytes in flight (16.8 MB over the GPU, past the 6-15 MB at which the
             // read probe peaks): waiting for every issued stage there took C5 7.50 -> 7.44 ms
-            if (D != 256 && nst - st - AHEAD - 1 >= NS - 2 - AHEAD) {
-                ESDA_WAIT_VM((NS - 2 - AHEAD) * DPW);
+            if (D != 256 && nst - st - 2 >= NS - 3) {
+                ESDA_WAIT_VM((NS - 3) * DPW);
             } else {
                 ESDA_WAIT_VM(0);
             }
         }
         lds_barrier();
-        if (st + NS - 1 < nst) dma(st + NS - 1, ring(std::integral_constant<int, (u + NS - 1) % NS>{}), (u + NS - 1) % NS);
-        // q8: widen stage st+3 (landed: this iteration's wait) for the next iterations
-        if constexpr (Q8) {
-            if (st + 3 < nst) convert(st + 3, ring(std::integral_constant<int, (u + 3) % NS>{}));
-        }
+        if (st + NS - 1 < nst) dma(st + NS - 1, ring(std::integral_constant<int, (u + NS - 1) % NS>{}));
         f32x4 sc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (RAW || !kLiveX || li < p.G) {
+        if (!kLiveX || li < p.G) {
             sc = xch[st & 1][0][lane];
 #pragma unroll
             for (int w = 1; w < NW; ++w) sc += xch[st & 1][w][lane];
         }
-        // V^T operands of this stage (plain kernels), read behind the exchange so that
+        // V^T operands of this stage, read behind the exchange so that
         // their latency hides under the softmax instead of following it
-        const unsigned char *vb = cbuf(st, uc) + VOFF;
-        short4v va[RAW ? 1 : DTW];
-        if constexpr (!RAW) {
+        const unsigned char *vb = ring(uc) + VOFF;
+        short4v va[DTW];
 #pragma unroll
-            for (int dt = 0; dt < DTW; ++dt)
-                va[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) short4v *) (vb + tr_off + 32 * dt));
-        }
+        for (int dt = 0; dt < DTW; ++dt)
+            va[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) short4v *) (vb + tr_off + 32 * dt));
         // The look-ahead work runs unconditionally (one basic block with the softmax, so
         // the two interleave): past the last stage it reads stale but in-bounds LDS and
         // writes exchange slots that are never read again.
-        if constexpr (RAW) {
-            qk_raw((st + 1) % 3, (st + 1) & 1, (st + 1) & 1, (u + 1) % NS);
-            load_raw(cbuf(st + 2, std::integral_constant<int, (u + 2) % NS>{}));
-            publish_ss((st + 2) % 3);
-            publish_tab(st + 2, st & 1);
-        } else {
-            qk_partial(ring(std::integral_constant<int, (u + 1) % NS>{}), (st + 1) & 1);
-        }
+        qk_partial(ring(std::integral_constant<int, (u + 1) % NS>{}), (st + 1) & 1);
         // Online softmax (log2 domain), identical in every wave; rows past the split
         // end (last stage only) and rows of another kv head of the group are masked.
         const int jt = j0 + st * RPP + jl;
@@ -899,48 +511,21 @@ void attend_kernel(AttendParams p) {
             const float mnew = fmaxf(m, tmax);
             const float corr = __builtin_amdgcn_exp2f(m - mnew);
             l *= corr;
-            if constexpr (Q8) bt *= corr;
 #pragma unroll
             for (int dt = 0; dt < DTW; ++dt) acc[dt] *= corr;
             m = mnew;
         }
         short4v pbs;
-        if constexpr (RAW) {
-            // V = kraw * rinv enters through the weight: P = bf16(e * rinv).  l adds the
-            // same rounded weight divided by rinv (ms * rinv = 1 / rinv), so numerator and
-            // denominator carry identical rounding and a dominant row is reproduced exactly.
-            // q8: the factor is scale * rinv (V enters as q) and the bias adds P * bias / scale.
-            const f32x4 ri = *reinterpret_cast<const f32x4 *>(&xr[st & 1][0][4 * lg]);
-            const f32x4 rn = *reinterpret_cast<const f32x4 *>(&xr[st & 1][1][4 * lg]);
-            f32x4 gm = {0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (Q8) gm = *reinterpret_cast<const f32x4 *>(&xr[st & 1][2][4 * lg]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float e = __builtin_amdgcn_exp2f(sc[r] - m);
-                const __bf16 pw = (__bf16) (e * ri[r]);
-                l += (float) pw * rn[r];
-                if constexpr (Q8) bt += (float) pw * gm[r];
-                pbs[r] = __builtin_bit_cast(short, pw);
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const __bf16 pr = (__bf16) __builtin_amdgcn_exp2f(sc[r] - m);
-                l += (float) pr;
-                pbs[r] = __builtin_bit_cast(short, pr);
-            }
+        for (int r = 0; r < 4; ++r) {
+            const __bf16 pr = (__bf16) __builtin_amdgcn_exp2f(sc[r] - m);
+            l += (float) pr;
+            pbs[r] = __builtin_bit_cast(short, pr);
         }
         // O^T (this wave's dims) += V^T . P^T
 #pragma unroll
-        for (int dt = 0; dt < DTW; ++dt) {
-            if constexpr (RAW) {
-                const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) short4v *) (vb + tr_off + 32 * dt));
-                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, pbs, acc[dt], 0, 0, 0);
-            } else {
-                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[dt], pbs, acc[dt], 0, 0, 0);
-            }
-        }
+        for (int dt = 0; dt < DTW; ++dt)
+            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[dt], pbs, acc[dt], 0, 0, 0);
     };
     for (int s0 = 0; s0 < nst; s0 += NS) unroll<NS>([&](auto uc) { stage(s0, uc); });
 
@@ -948,7 +533,7 @@ void attend_kernel(AttendParams p) {
     // into its cache row (bit-exact).  Its own DMA reads that row from k_new / v_new and
     // no other workgroup reads it; the copy runs after this workgroup's ring has
     // drained, so no outstanding load is counted against the ring's waits.
-    if (!Q8 && append && j1 == sv.nvis) {
+    if (append && j1 == sv.nvis) {
         for (int pr = wave; pr < pk; pr += NW) {  // wave pr copies kv head pr of the group
             const size_t row = (size_t) pr * p.head_stride + (size_t) sv.newrow * D;
             for (int c = lane; c < D / 8; c += 64) {
@@ -964,13 +549,6 @@ void attend_kernel(AttendParams p) {
     // Partial of this split: every wave holds the same (m, l) and its own dim slice.
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    if constexpr (Q8) {
-        // the bias part of PV is the same for every dim of a head
-        bt += __shfl_xor(bt, 16);
-        bt += __shfl_xor(bt, 32);
-#pragma unroll
-        for (int dt = 0; dt < DTW; ++dt) acc[dt] += bt;
-    }
     if (direct) {
         // The only segment of this (sequence, kv head): normalise here, with the merge's
         // arithmetic (acc * (1 / l), then bf16); the merge skips this pair.
@@ -1010,8 +588,7 @@ void attend_kernel(AttendParams p) {
 
 // ------------------------------------------------- raw-K attend with wave-private rings
 //
-// Raw-K decode (ESDecodeAttn.mm:17-117) when the caller passes the precomputed rotary table
-// -- the ES layer's path.  A workgroup serves one kv head (a contiguous run of its rows, as
+// Raw-K decode (ESDecodeAttn.mm:17-117).  A workgroup serves one kv head (a contiguous run of its rows, as
 // the composite kernel's) with four waves, one per SIMD.  Each wave owns whole 16-row stages
 // (16 consecutive positions) over the full 512-dim head, in turn: wave w takes stages w,
 // w + 4, w + 8, ... of a segment.  It streams their rows through two LDS slots of its own and
@@ -1028,7 +605,11 @@ void attend_kernel(AttendParams p) {
 //     hands every lane the dims it supplied; one multiply by rinv, the rotation and the
 //     bf16 rounding remain per element.  The rotary partners (d, d + 256), d < 64, sit in
 //     one lane (k-steps 0, 1 and 8, 9); their bf16 cos / sin come from the table rows,
-//     whose buffer takes the next stage's table rows once the rotary k-steps have read it;
+//     whose buffer takes the next stage's table rows once the rotary k-steps have read it,
+//     or, when the caller passes no table, are computed by the lane that uses them (16 per
+//     lane and stage, ~430 VALU instructions: 131072 rows x 4 heads raw 105.7 us a step
+//     against 95.8 with the table and 160.6 by an 8-wave kernel that shared a computed
+//     table through LDS; q8 118.4, 95.3 and 207.5);
 //   - scores the kv head's query heads (up to 16: the MFMA's N dimension, zero-padded) with
 //     16 MFMAs, runs its own online softmax, and accumulates O^T[512 x 16 heads] with 32
 //     MFMAs over V = kraw read back by transpose reads, rinv folded into the weight:
@@ -1060,16 +641,16 @@ __device__ __forceinline__ constexpr bool rot_step(int kk) { return (kk & 7) < 2
 // with the generic threshold of 8 about half of all stages would rescale.
 constexpr float kRawRescaleSlack = 64.0f;
 
-template <bool Q8>
+template <bool Q8, bool TABLE>
 struct WRing {
     static constexpr int ROWS = Q8 ? 8 * kBlk : 16 * kBlk;  // a stage's 16 rows (q8: two per block)
     static constexpr int SB = Q8 ? 128 : 0;                  // q8: 16 scales, 16 biases
     static constexpr int SLOT = ROWS + SB;
     static constexpr int STG = Q8 ? 16 * kBlk : 0;           // q8: the bf16 V tile
-    static constexpr int TAB = 4 * kBlk;                     // the stage's 16 cos/sin table rows (swizzled)
+    static constexpr int TAB = TABLE ? 4 * kBlk : 0;         // the stage's 16 cos/sin table rows (swizzled)
     static constexpr int WAVE = 2 * SLOT + STG + TAB;        // one wave's LDS: two slots, the V tile, the table
     static constexpr int MERGE = kWaves * 16 * 516 * 4;      // end-of-segment merge area (aliases the rings)
-    static_assert(kWaves * WAVE >= MERGE, "the merge area fits in the rings");
+    static constexpr int LDS = kWaves * WAVE > MERGE ? kWaves * WAVE : MERGE;
 };
 
 // DMA of LDS blocks I .. N-1 of an interior stage: block i is 1 KiB of memory at
@@ -1084,11 +665,11 @@ __device__ __forceinline__ void ring_blocks(const uint64_t *base, unsigned voff,
     }
 }
 
-template <bool Q8>
+template <bool Q8, bool TABLE>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(1, 1)))
 void raw_attend_kernel(AttendParams p) {
-    using W = WRing<Q8>;
-    __shared__ __attribute__((aligned(16))) unsigned char wlds[kWaves * W::WAVE];
+    using W = WRing<Q8, TABLE>;
+    __shared__ __attribute__((aligned(16))) unsigned char wlds[W::LDS];
     // per-wave row factors of the stage being computed (the softmax's rows 4lg .. 4lg + 3):
     // [0] rinv (q8: scale * rinv), [1] its inverse, [2] (q8) bias / scale
     __shared__ __attribute__((aligned(16))) float xf[kWaves][3][16];
@@ -1100,12 +681,17 @@ void raw_attend_kernel(AttendParams p) {
     // q8: the k-norm weights in fp32, read per k-step (the lanes of a lane group read the
     // same 32 bytes); 128 of them per lane would not fit in registers beside O^T and Q^T.
     __shared__ __attribute__((aligned(16))) float kwl[Q8 ? kRawDim : 1];
+    // no table: the rotary frequencies, read back per stage
+    __shared__ __attribute__((aligned(16))) float invl[TABLE ? 1 : kRopePairs];
+    if constexpr (!TABLE) {
+        if (tid < kRopePairs) invl[tid] = p.inv_freq[tid];
+    }
     if constexpr (Q8) {
         const unsigned t = reinterpret_cast<const unsigned *>(p.kw)[tid];
         kwl[2 * tid] = bf16_lo(t);
         kwl[2 * tid + 1] = bf16_hi(t);
-        __syncthreads();
     }
+    if constexpr (Q8 || !TABLE) __syncthreads();
     // Raw: the A operands of the x * kw products, diag(kw) over 16 dims.  For k-step kk and half
     // hh the B operand is the lane's own dims kdim(kk, lg) + 4hh .. + 3 of row li; lane
     // (li, lg) then holds kw of dim kdim(kk, lg) + 4hh + (li & 3) at slot li & 3 when
@@ -1289,7 +875,7 @@ void raw_attend_kernel(AttendParams p) {
         const int st0 = wave;
         if (st0 < nst) {
             dma_rows(st0, wl);
-            dma_tab(st0);
+            if constexpr (TABLE) dma_tab(st0);
         }
 
         float m = -INFINITY, l = 0.0f;
@@ -1312,8 +898,24 @@ void raw_attend_kernel(AttendParams p) {
             // Scores S^T[16 rows x 16 heads] of K = bf16(rope(x * rinv * kw)) (q8: x = q * scale
             // + bias), rounded where ESDecodeAttn.mm:51-93 rounds it.
             f32x4 sp0 = {0.0f, 0.0f, 0.0f, 0.0f}, sp1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            // cos / sin of row li's position for the rotary pairs this lane holds
+            // cos / sin of row li's position for the rotary pairs this lane holds: from the
+            // table, or computed (rope_table_kernel's arithmetic; the lanes of a stage need
+            // 16 x 64 pairs, so each computes the 16 it uses)
             auto load_tab = [&](u32x4 (&tab)[4]) {
+                if constexpr (!TABLE) {
+                    const float t = (float) (sv.first + min(j0 + 16 * st + li, j1 - 1));
+#pragma unroll
+                    for (int c4 = 0; c4 < 4; ++c4) {
+                        const f32x4 f = *reinterpret_cast<const f32x4 *>(invl + 32 * (c4 >> 1) + 8 * lg + 4 * (c4 & 1));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float sn, cs;
+                            sincos_f32(t * f[e], sn, cs);
+                            tab[c4][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{cs, sn}, bf16x2));
+                        }
+                    }
+                    return;
+                }
                 const int bt2 = li >> 2, rib = li & 3;  // row li: position li of the stage
 #pragma unroll
                 for (int c4 = 0; c4 < 4; ++c4) {
@@ -1464,8 +1066,10 @@ void raw_attend_kernel(AttendParams p) {
             }
             // the table buffer is read (the rotary k-steps above): the next stage's rows may land
             if (st + kWaves < nst) {
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                dma_tab(st + kWaves);
+                if constexpr (TABLE) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    dma_tab(st + kWaves);
+                }
                 if constexpr (!Q8) dma_rows_part(st + kWaves, nsl, std::integral_constant<int, 2>{});
             }
 #pragma unroll
@@ -1837,7 +1441,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t *src,
 }
 
 // Rotary cos/sin table for raw-K decode: entry (t, f) = bf16 cos | bf16 sin << 16 of the
-// fp32 angle t * inv_freq[f], t < rows, f < 64 -- publish_tab's arithmetic.
+// fp32 angle t * inv_freq[f], t < rows, f < 64 -- what raw_attend_kernel computes without a table.
 __global__ __launch_bounds__(256) void rope_table_kernel(const float *inv_freq, long long n, unsigned *tab) {
     const long long i = (long long) blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
@@ -2067,14 +1671,10 @@ int make_plan(const esda_decode_desc *d, Plan *pl, bool raw = false) {
 template <int D>
 constexpr int ring_waves() { return D == 256 ? kWaves256 : 4; }
 
-// Raw mode: 8 waves, two per SIMD, so one wave's dependency stalls overlap the other's
-// reconstruction work.
-constexpr int kRawWaves = 8;
-
-template <int D, bool SHARED, bool RAW = false, bool Q8 = false, int OCC = 1>
+template <int D, bool SHARED, int OCC = 1>
 hipError_t launch_attend(const AttendParams &ap, dim3 grid, hipStream_t st) {
-    constexpr int NW = RAW ? kRawWaves : ring_waves<D>();
-    hipLaunchKernelGGL((attend_kernel<D, SHARED, NW, RAW, Q8, OCC>), grid, dim3(64 * NW), 0, st, ap);
+    constexpr int NW = ring_waves<D>();
+    hipLaunchKernelGGL((attend_kernel<D, SHARED, NW, OCC>), grid, dim3(64 * NW), 0, st, ap);
     return hipGetLastError();
 }
 
@@ -2091,10 +1691,10 @@ hipError_t dispatch_attend(int D, bool shared, const AttendParams &ap, dim3 grid
     switch (D) {
         case 128: return shared ? launch_attend<128, true>(ap, grid, st) : launch_attend<128, false>(ap, grid, st);
         case 256:
-            return shared ? launch_attend<256, true, false, false, O256>(ap, grid, st)
-                          : launch_attend<256, false, false, false, O256>(ap, grid, st);
+            return shared ? launch_attend<256, true, O256>(ap, grid, st)
+                          : launch_attend<256, false, O256>(ap, grid, st);
         default:
-            return shared ? launch_attend<512, true, false, false, O512>(ap, grid, st)
+            return shared ? launch_attend<512, true, O512>(ap, grid, st)
                           : launch_attend<512, false>(ap, grid, st);
     }
 }
@@ -2158,17 +1758,13 @@ int run_stages(const esda_decode_desc *d, const Plan &pl, const AttendParams &ap
         hipError_t e;
         if (mode == 0) {
             e = dispatch_attend(d->head_dim, d->kv_shared != 0, ap, grid, st);
-        } else if (ap.rope_tab) {
-            // with the precomputed cos/sin table (the ES layer's form): the wave-private-ring
-            // kernel, one kv head per workgroup
-            if (mode == 1) hipLaunchKernelGGL(raw_attend_kernel<false>, grid, dim3(64 * kWaves), 0, st, ap);
-            else hipLaunchKernelGGL(raw_attend_kernel<true>, grid, dim3(64 * kWaves), 0, st, ap);
-            e = hipGetLastError();
-        } else if (mode == 1) {
-            // without a table the 8-wave kernel computes its cos/sin per stage
-            e = launch_attend<kRawDim, true, true>(ap, grid, st);
         } else {
-            e = launch_attend<kRawDim, true, true, true>(ap, grid, st);
+            const dim3 block(64 * kWaves);
+            if (mode == 1 && ap.rope_tab) hipLaunchKernelGGL((raw_attend_kernel<false, true>), grid, block, 0, st, ap);
+            else if (mode == 1) hipLaunchKernelGGL((raw_attend_kernel<false, false>), grid, block, 0, st, ap);
+            else if (ap.rope_tab) hipLaunchKernelGGL((raw_attend_kernel<true, true>), grid, block, 0, st, ap);
+            else hipLaunchKernelGGL((raw_attend_kernel<true, false>), grid, block, 0, st, ap);
+            e = hipGetLastError();
         }
         if (e != hipSuccess) return hip_fail(e, "attend_kernel launch");
     }

@@ -164,8 +164,8 @@ typedef struct esda_raw_args {
     void *workspace;         /* esda_decode_raw_workspace_size bytes; first 256 zeroed once */
     size_t workspace_bytes;
     const void *rope_table;  /* optional, NULL: computed in the kernel.  [rope_table_rows][64]
-                                u32 from esda_rope_table (cos / sin of row*inv_freq[d]);
-                                read where two kv heads share a workgroup              */
+                                u32 from esda_rope_table (cos / sin of row*inv_freq[d]):
+                                the same values and outputs, read instead of computed   */
     int32_t rope_table_rows; /* >= cap when rope_table is set                          */
 } esda_raw_args;
 
