@@ -1338,11 +1338,12 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(MergeParams p) {
     }
 }
 
-// Merge for pairs of few splits (balanced shares): one thread per (sequence,
+// Merge for pairs of few splits: one thread per (sequence,
 // query head, 4 output dims), no barriers.  Splits are read 8 at a time -- the loads of
 // a chunk issue together, so up to 8 splits cost one memory round trip -- with the
 // running max raised per chunk (same result as merge_kernel up to summation order).
 constexpr int kMergeRowsThreads = 256;
+constexpr int kMergeShares = 6;  // balanced shares per pair from which merge_kernel is the faster merge
 constexpr int kMergeRowsChunk = 8;
 
 __global__ __launch_bounds__(kMergeRowsThreads) void merge_rows_kernel(MergeParams p) {
@@ -1789,18 +1790,23 @@ int run_stages(const esda_decode_desc *d, const Plan &pl, const AttendParams &ap
         mp.W = pl.W;
         mp.S = pl.S;
         mp.chunk = pl.chunk;
-        if (pl.balanced || pl.S <= kMergeRowsChunk) {
-            // Balanced shares give each pair a few splits: thread-per-output merge (C5's
-            // global layers: 11 -> 4.4 us), as do grids of at most kMergeRowsChunk splits
-            // (one memory round trip per thread).  Larger grids keep merge_kernel, whose
-            // workgroups reduce 16 split groups side by side (at C1's 16 splits over 8 pairs
-            // the rows kernel would run 4 workgroups and two round trips: 9.0 -> 11.8 us a step).
+        // Partials per pair: a grid's S, or about W / pairs + 1 of the balanced shares.
+        const long long pairs = (long long) d->batch * d->num_kv_heads / pl.pk;
+        if (pl.balanced ? pl.W < kMergeShares * pairs : pl.S <= kMergeRowsChunk) {
+            // A few splits per pair: the thread-per-output merge, one memory round trip per
+            // kMergeRowsChunk of them (C5's global layers, 128 pairs of 3 partials: 11 -> 4.4
+            // us).  With more, merge_kernel's workgroups reduce 16 split groups side by side:
+            // at C1's 16 splits over 8 pairs the rows kernel takes two round trips (9.0 ->
+            // 11.8 us a step), and on balanced shares (step us, rows / merge_kernel): 8 pairs of
+            // 32 partials 46.1 / 30.0, 16 of 16 47.7 / 38.4, 32 of 8 41.6 / 38.7, 40 of 6.4
+            // 50.4 / 49.6, 48 of 5.3 51.0 / 50.8, 64 of 4 39.5 / 42.5.
             const int threads = d->num_q_heads * (d->head_dim / 4);
             dim3 grid((threads + kMergeRowsThreads - 1) / kMergeRowsThreads, d->batch);
             hipLaunchKernelGGL(merge_rows_kernel, grid, dim3(kMergeRowsThreads), 0, st, mp);
         } else {
             dim3 grid(d->head_dim / kMergeDims, d->num_q_heads, d->batch);
-            if (pl.S <= kMergeGroups * 4)
+            // (balanced: room for a pair of twice the average partials; longer ones are looped over)
+            if (pl.balanced ? 2LL * pl.W <= kMergeGroups * 4 * pairs : pl.S <= kMergeGroups * 4)
                 hipLaunchKernelGGL(merge_kernel<4>, grid, dim3(kMergeThreads), 0, st, mp);
             else
                 hipLaunchKernelGGL(merge_kernel<16>, grid, dim3(kMergeThreads), 0, st, mp);
