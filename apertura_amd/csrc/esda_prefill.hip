@@ -69,12 +69,17 @@ struct PrefillParams {
     int kh;                  // 1: the two wave groups split each tile's stages (even / odd)
 };
 
+// Query row r of a GQA group's rows -> its position in the chunk (r % G is its head).  At
+// most 2^24 tiles of 256 rows (plan_prefill), so 32-bit divisions: the 64-bit ones took
+// ~4,000 of a workgroup's first 13,000 cycles.
+__host__ __device__ inline unsigned position_of(long long r, int G) { return (unsigned) r / (unsigned) G; }
+
 // Keys [j0, j1) that some row of query tile `tile` (QT rows) can see.
 __host__ __device__ inline void tile_keys(const PrefillParams &p, int tile, int QT, int &j0, int &j1) {
     const long long rows = (long long) p.Sq * p.G;
     const long long r0 = (long long) tile * QT;
     const long long r1 = (r0 + QT < rows ? r0 + QT : rows) - 1;
-    const long long qa0 = p.q_pos0 + r0 / p.G, qa1 = p.q_pos0 + r1 / p.G;
+    const long long qa0 = p.q_pos0 + position_of(r0, p.G), qa1 = p.q_pos0 + position_of(r1, p.G);
     long long lo = p.window > 0 ? qa0 - p.window + 1 - p.k_pos0 : 0;
     long long hi = qa1 - p.k_pos0 + 1;
     if (lo < 0) lo = 0;
@@ -189,7 +194,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
             for (int qb = 0; qb < QB; ++qb)
                 if (qvalid(qb)) {
                     const long long gr = qrow(qb);
-                    const long long row = (gr / p.G) * p.Hq + kvh * p.G + gr % p.G;
+                    const unsigned qi = position_of(gr, p.G);
+                    const long long row = (long long) qi * p.Hq + kvh * p.G + (int) ((unsigned) gr - qi * p.G);
                     *reinterpret_cast<f32x2 *>(p.part_ml + 2 * ((long long) split * nrows + row)) =
                         f32x2{-INFINITY, 0.0f};
                 }
@@ -203,8 +209,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         const long long gr = qrow(qb);
-        const uint16_t *qr = p.q + (size_t) (kvh * p.G + gr % p.G) * p.q_hs + (size_t) (gr / p.G) * p.q_rs + lg * 8;
-        qabs[qb] = p.q_pos0 + (int) (gr / p.G);
+        const unsigned qi = position_of(gr, p.G);
+        const uint16_t *qr = p.q + (size_t) (kvh * p.G + (int) ((unsigned) gr - qi * p.G)) * p.q_hs +
+                             (size_t) qi * p.q_rs + lg * 8;
+        qabs[qb] = p.q_pos0 + (int) qi;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             u32x4 w = qvalid(qb) ? *reinterpret_cast<const u32x4 *>(qr + ks * 32) : u32x4{0u, 0u, 0u, 0u};
@@ -277,8 +285,9 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
         if (lane < 2) *(lds_flag *) (xch + lane * XPAR + kWaves * XP + wave * 4) = 0u;
     }
     // Positions of the tile's first and last rows (the host keeps positions below 2^31).
-    const int qa_min = p.q_pos0 + (int) ((long long) tile * QT / p.G);
-    const int qa_max = p.q_pos0 + (int) (((long long) tile * QT + QT < nq ? (long long) tile * QT + QT : nq) - 1) / p.G;
+    const int qa_min = p.q_pos0 + (int) position_of((long long) tile * QT, p.G);
+    const int qa_max = p.q_pos0 +
+                       (int) position_of(((long long) tile * QT + QT < nq ? (long long) tile * QT + QT : nq) - 1, p.G);
 
     // S^T[keys x queries] of a stage: s[h][qb] covers keys 16h + 4lg + r of query column li.
     struct Scores {
@@ -547,7 +556,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
         const long long gr0 = (long long) tile * QT + br + li;
         if (gr0 >= nq) continue;
         const long long gr = gr0;
-        const int qi = (int) (gr / p.G), qh = kvh * p.G + (int) (gr % p.G);
+        const int qi = (int) position_of(gr, p.G), qh = kvh * p.G + (int) ((unsigned) gr - (unsigned) qi * p.G);
         const long long row = (long long) qi * p.Hq + qh;
         const int d0 = 16 * DW * hd;  // the wave's first O^T dim
         if (p.splits == 1) {
