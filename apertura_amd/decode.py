@@ -106,8 +106,12 @@ def _check_row_base(step, row_base: torch.Tensor | None) -> None:
 
 
 def _stream_ptr(stream) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    """The HIP stream of `stream`, or of the calling thread's current stream.  The handle
+    alone: torch.cuda.current_stream() builds a Stream object, 2.8 us against 0.2 of a call
+    whose two launches take 5.6."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def decode_step(step: DecodeStep, q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor | None,

@@ -68,8 +68,11 @@ class PrefillStep:
 
 
 def prefill_workspace_bytes(step: PrefillStep) -> int:
+    return _workspace_bytes(step.desc())
+
+
+def _workspace_bytes(d: PrefillDesc) -> int:
     n = ctypes.c_size_t(0)
-    d = step.desc()
     check(lib().esda_prefill_workspace_size(ctypes.byref(d), ctypes.byref(n)))
     return int(n.value)
 
@@ -89,21 +92,18 @@ def prefill(step: PrefillStep, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
         out = torch.empty((step.seq_q, step.num_q_heads, D), dtype=bf, device=q.device)
     d = step.desc()
     # the extent each tensor must cover (elements), checked before the pointers go down
-    need = {
-        "q": (step.num_q_heads - 1) * d.q_head_stride + (step.seq_q - 1) * d.q_row_stride + D,
-        "k": (step.num_kv_heads - 1) * d.kv_head_stride + step.seq_k * D,
-        "out": (step.seq_q - 1) * d.out_row_stride + (step.num_q_heads - 1) * d.out_head_stride + D,
-    }
-    for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
+    kv = (d.num_kv_heads - 1) * d.kv_head_stride + d.seq_k * D
+    for name, t, need in (("q", q, (d.num_q_heads - 1) * d.q_head_stride + (d.seq_q - 1) * d.q_row_stride + D),
+                          ("k", k, kv), ("v", v, kv),
+                          ("out", out, (d.seq_q - 1) * d.out_row_stride + (d.num_q_heads - 1) * d.out_head_stride + D)):
         if t.dtype != bf or not t.is_cuda:
             raise ValueError(f"{name} must be a bf16 GPU tensor")
-        avail = t.untyped_storage().nbytes() // 2 - t.storage_offset()
-        if avail < need["k" if name == "v" else name]:
+        if t.untyped_storage().nbytes() // 2 - t.storage_offset() < need:
             raise ValueError(f"{name} is smaller than the description's extent")
-    nbytes = prefill_workspace_bytes(step)
+    nbytes = _workspace_bytes(d)
     if nbytes and (workspace is None or workspace.numel() * workspace.element_size() < nbytes):
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-    a = PrefillArgs(_dev_ptr(q), _dev_ptr(k), _dev_ptr(v), _dev_ptr(out),
+    a = PrefillArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                     _dev_ptr(workspace) if nbytes else None, nbytes)
     check(lib().esda_prefill_stages(ctypes.byref(d), ctypes.byref(a), int(stages), _stream_ptr(stream)))
     return out
