@@ -67,6 +67,7 @@ struct PrefillParams {
     int tiles, splits, kps;  // query tiles per kv head, key splits, keys per split
     float scale_log2e;
     int kh;                  // 1: the two wave groups split each tile's stages (even / odd)
+    int part_nt;             // 1: partials stored non-temporal
 };
 
 // Query row r of a GQA group's rows -> its position in the chunk (r % G is its head).  At
@@ -570,8 +571,16 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
             }
         } else {
             float *pa = p.part_acc + ((long long) split * nrows + row) * D + d0 + 4 * lg;
+            if (p.part_nt) {
+                // (the barriers keep the two branches' stores from being merged into plain ones)
+                asm volatile("" ::: "memory");
 #pragma unroll
-            for (int dt = 0; dt < DW; ++dt) *reinterpret_cast<f32x4 *>(pa + 16 * dt) = acc[nb][dt];
+                for (int dt = 0; dt < DW; ++dt) __builtin_nontemporal_store(acc[nb][dt], reinterpret_cast<f32x4 *>(pa + 16 * dt));
+                asm volatile("" ::: "memory");
+            } else {
+#pragma unroll
+                for (int dt = 0; dt < DW; ++dt) *reinterpret_cast<f32x4 *>(pa + 16 * dt) = acc[nb][dt];
+            }
             if (lg == 0 && nb < QB)  // (m, l) from the block's owner
                 *reinterpret_cast<f32x2 *>(p.part_ml + 2 * ((long long) split * nrows + row)) = f32x2{m[nb < QB ? nb : 0], l[nb < QB ? nb : 0]};
         }
@@ -887,9 +896,14 @@ float makespan(int Hkv, const Tiling &t, F &&pieces) {
     return most * share;
 }
 
-// Splitting adds a dependent launch (us) and D fp32 per row and split, written by the
-// attention kernel and read by the merge (us per byte).
-constexpr float kSplitLaunch = 6.5f, kPartialByte = 3.1e-7f;
+// Splitting adds a dependent launch and D fp32 per row and split, written by the attention
+// kernel and read by the merge.  Few partials are stored non-temporal: the merge reads them
+// from other XCDs, and the launch boundary then has no dirty lines to write back (64 local
+// queries in 4 splits, 8 MB: 19.5 -> 17.9 us; 200 in 2, 13 MB: 28.3 -> 25.2).  Past the XCDs'
+// L2s together (8 x 4 MB) the write-back overlaps the kernel, and waiting for memory costs
+// more: 32 MB 46.7 -> 45.7 us, 40 MB 43.7 both ways, 48 MB 42.2 -> 46.4, 64 MB 42.2 -> 54.0.
+constexpr float kPartNtBytes = 36.0e6f;
+float split_cost(float part_bytes) { return 5.0f + 3.1e-7f * part_bytes; }  // us
 constexpr int kMaxRounds = 3;  // split plans of more workgroups per CU only add partials
 
 // Validates a description and fills the kernel parameters' shape fields and plan.
@@ -963,7 +977,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         }
         auto consider = [&](int per) {  // per: stages per split
             const int splits = (most + per - 1) / per;
-            float us = splits > 1 ? kSplitLaunch + kPartialByte * 4.0f * D * (float) rows * d->num_kv_heads * splits : 0.0f;
+            float us = splits > 1 ? split_cost(4.0f * D * (float) rows * d->num_kv_heads * splits) : 0.0f;
             if (us + t.wg + per * t.stage >= best) return splits;
             if (few)
                 us += makespan(d->num_kv_heads, t, [&](auto &&piece) {
@@ -996,6 +1010,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         return fail(ESDA_ERR_INVALID_ARGUMENT, "esda_prefill: too many key splits");
     p->kps = kps;
     p->splits = (int) std::max<long long>(1, splits);
+    p->part_nt = 4.0f * D * p->Sq * p->Hq * p->splits <= kPartNtBytes;
     return ESDA_OK;
 }
 
