@@ -712,10 +712,6 @@ struct RawKvParams {
 
 __device__ __forceinline__ float bf16r(float x) { return (float) (__bf16) x; }
 
-// Callers' rows need only their element's alignment.
-typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef unsigned u32x2_a1 __attribute__((ext_vector_type(2), aligned(1)));
-
 template <int D, bool Q8, int HG>
 __global__ __launch_bounds__(256) void raw_prefill_kv_kernel(RawKvParams p) {
 #pragma clang fp contract(off)  // every rounding point as written (no fused multiply-add)
