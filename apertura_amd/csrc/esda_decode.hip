@@ -1156,16 +1156,20 @@ void raw_attend_kernel(AttendParams p) {
         lds_barrier();
         float *const accb = reinterpret_cast<float *>(wlds);          // [wave][head][516]
         float *const mlb = &xf[0][0][0];                               // [wave][2][16] (m, l)
+        // Live heads only: at most 8 of them take 32 threads each, more take 16.
+        if (li < p.G) {
 #pragma unroll
-        for (int dt = 0; dt < 32; ++dt)
-            *reinterpret_cast<f32x4 *>(accb + (wave * 16 + li) * 516 + 16 * dt + 4 * lg) = acc[dt];
+            for (int dt = 0; dt < 32; ++dt)
+                *reinterpret_cast<f32x4 *>(accb + (wave * 16 + li) * 516 + 16 * dt + 4 * lg) = acc[dt];
+        }
         if (lg == 0) {
             mlb[wave * 32 + li] = m;
             mlb[wave * 32 + 16 + li] = l;
         }
         lds_barrier();
         {
-            const int h = tid >> 4, d4 = tid & 15;  // head h, dims 4 d4 + 64 k
+            const int lt = p.G <= 8 ? 5 : 4;  // log2 of the threads per head
+            const int h = tid >> lt, d4 = tid & ((1 << lt) - 1);  // head h, dims 4 d4 + (4 << lt) k
             float mw[kWaves], M = -INFINITY;
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
@@ -1182,9 +1186,8 @@ void raw_attend_kernel(AttendParams p) {
                 const size_t hq = (size_t) b * p.Hq + (size_t) kvh * p.G + h;
                 const size_t pidx = slot * p.G + h;
                 const float inv = 1.0f / L;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int d = 4 * d4 + 64 * k;
+#pragma unroll 4
+                for (int d = 4 * d4; d < kRawDim; d += 4 << lt) {
                     f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                     for (int w = 0; w < kWaves; ++w) o += *reinterpret_cast<const f32x4 *>(accb + (w * 16 + h) * 516 + d) * cw[w];
