@@ -966,7 +966,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         for (int i = 0; i < (int) tiles; ++i) {
             int a, b;
             tile_keys(*p, (int) tiles - 1 - i, QT, a, b);
-            const int n = (b - a + kStageKeys - 1) / kStageKeys;
+            const int n = (int) (((long long) b - a + kStageKeys - 1) / kStageKeys);
             if (few) nst[i] = n;
             most = std::max(most, n);
             total += t.wg + n * t.stage;
@@ -974,13 +974,13 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         auto consider = [&](int per) {  // per: stages per split
             const int splits = (most + per - 1) / per;
             float us = splits > 1 ? split_cost(4.0f * D * (float) rows * d->num_kv_heads * splits) : 0.0f;
-            if (us + t.wg + per * t.stage >= best) return splits;
-            if (few)
+            if (us + t.wg + std::min(per, most) * t.stage >= best) return splits;
+            if (few && tiles * splits <= 2LL * kMaxRounds * kTargetGroups)
                 us += makespan(d->num_kv_heads, t, [&](auto &&piece) {
                     for (int i = 0; i < (int) tiles; ++i)
                         for (int j = 0; j < nst[i]; j += per) piece(std::min(per, nst[i] - j));
                 });
-            else  // many rounds: the CUs stay busy but for the end of the last
+            else  // many workgroups: the CUs stay busy but for the end of the last round
                 us += (float) (total * d->num_kv_heads / kTargetGroups) + 0.5f * (t.wg + most * t.stage);
             if (us < best) {
                 best = us;
@@ -993,7 +993,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
             return splits;
         };
         if (d->split_keys > 0) {
-            consider(few ? d->split_keys / kStageKeys : most);
+            consider(d->split_keys / kStageKeys);
         } else {
             consider(most);
             for (int s = 2; s <= most && groups * s <= kMaxRounds * kTargetGroups;)

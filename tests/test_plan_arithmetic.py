@@ -38,3 +38,38 @@ def test_planted_prefix_table_bug_is_caught(tmp_path):
     exe = _build(tmp_path, "PLANT_TABLE_BUG")
     r = subprocess.run([str(exe), "64"], capture_output=True, text=True, timeout=600)
     assert r.returncode != 0 and "table[256] never written" in r.stdout, r.stdout[-2000:]
+
+
+def _prefill_bytes(Hq, Hkv, D, Sq, Sk, q_pos0, k_pos0=0, window=0, split_keys=0):
+    from apertura_amd.prefill import PrefillStep, prefill_workspace_bytes
+    return prefill_workspace_bytes(PrefillStep(Hq, Hkv, D, Sq, Sk, q_pos0, k_pos0, window, split_keys=split_keys,
+                                               kv_head_stride=Sk * D))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,Sq,past,splits", [
+    (32, 4, 512, 333, 5600, 3),    # 84 tiles: 252 workgroups, not 336
+    (32, 4, 512, 200, 8056, 4),    # 52 tiles: 208
+    (32, 4, 512, 512, 15872, 2),   # 128 tiles: 256
+    (32, 4, 512, 770, 0, 1),       # 196 fresh tiles: unsplit
+    (32, 4, 512, 4096, 0, 1),      # four rounds of tiles
+    (8, 4, 256, 17, 10, 1),        # one stage
+])
+def test_prefill_plan_fills_whole_rounds(Hq, Hkv, D, Sq, past, splits):
+    """Automatic key splits by the workspace they ask for (D fp32 and (m, l) per row and split)."""
+    n = _prefill_bytes(Hq, Hkv, D, Sq, past + Sq, past)
+    assert n == (0 if splits == 1 else splits * Sq * Hq * (D * 4 + 8) + 256)
+
+
+def test_prefill_plan_of_extreme_forced_splits_is_quick():
+    """Forced splits are planned without walking them: the largest accepted count, a count
+    past the limit (refused), and one split longer than the keys."""
+    import time
+
+    from apertura_amd import EsdaError
+    t0 = time.perf_counter()
+    n = 65535 * 32
+    assert _prefill_bytes(16, 8, 256, 64, n, n - 64, split_keys=32) == 65535 * 64 * 16 * (256 * 4 + 8) + 256
+    with pytest.raises(EsdaError):
+        _prefill_bytes(16, 8, 256, 64, 2 ** 30, 2 ** 30 - 64, split_keys=32)
+    assert _prefill_bytes(16, 8, 256, 2 ** 20, 2 ** 20, 0, split_keys=2 ** 30) == 0
+    assert time.perf_counter() - t0 < 2.0
