@@ -24,6 +24,7 @@
 //                       straight from the score registers (the 32 keys are ordered so
 //                       that the score layout is the B-operand layout).  O^T stays in
 //                       registers (D/16 x QB tiles: QB * D / 16 accumulators per lane).
+//                       Four waves and 64-row tiles for short chunks at D = 512.
 //   prefill_kernel<256, 1, true>  the same with 64-row tiles whose even and odd stages go
 //                       to the two wave groups (waves 0-3 and 4-7 on the same query
 //                       blocks), folded together through LDS at the end: short chunks
@@ -63,10 +64,11 @@ struct PrefillParams {
     float *part_ml;    // [splits][Sq * Hq][2]
     long long q_hs, q_rs, kv_hs, o_rs, o_hs;
     int Hq, Hkv, G, Sq, Sk, q_pos0, k_pos0, window;
-    int qb;                  // 16-query blocks per wave (query tile: 128 qb rows, 64 with kh)
+    int qb;                  // 16-query blocks per wave
     int tiles, splits, kps;  // query tiles per kv head, key splits, keys per split
     float scale_log2e;
     int kh;                  // 1: the two wave groups split each tile's stages (even / odd)
+    int nw;                  // waves per workgroup (query tile: 16 qb nw rows, half of it with kh)
     int part_nt;             // 1: partials stored non-temporal
 };
 
@@ -138,11 +140,11 @@ struct PRing {
 // parity only after reading its partner's next flag, which the partner writes after reading
 // this stage's P^T.  Used by the K = V kernel at D = 512 (p512gs 436 -> 422 us on one box);
 // with separate K and V -- one stage per barrier -- it measured 1-3% slower and is not used.
-template <int D, int QB, bool KH = false, bool SH = false, bool S2 = false, bool PS = false>
-__global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p) {
+template <int D, int QB, bool KH = false, bool SH = false, bool S2 = false, bool PS = false, int NW = kWaves>
+__global__ __launch_bounds__(64 * NW, 1) void prefill_kernel(PrefillParams p) {
     static_assert(!S2 || !KH, "two stages per iteration: all waves on both");
     static_assert(!PS || (QB == 1 && !KH), "pair split: one block per wave, every wave on every stage");
-    constexpr int NQW = KH ? kWaves / 2 : kWaves;  // waves with distinct query blocks
+    constexpr int NQW = KH ? NW / 2 : NW;  // waves with distinct query blocks
     constexpr int NSL = KH || S2 ? 4 : 2;          // ring stages per tensor
     constexpr int SPI = KH || S2 ? 2 : 1;          // stages per iteration (KH: one per wave group)
     using R = PRing<D, NSL, SH ? 1 : 2>;
@@ -155,8 +157,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
     // PS exchange, per stage parity: each wave's P^T (16 B per lane) and rescale factors
     // (4 B per lane), then one flag per wave; after both parities, each wave's row sums.
     constexpr int XP = 64 * 16 + 64 * 4;
-    constexpr int XPAR = kWaves * XP + kWaves * 4;
-    __shared__ __attribute__((aligned(16))) unsigned char xch[PS ? 2 * XPAR + kWaves * 16 * 4 : 16];
+    constexpr int XPAR = NW * XP + NW * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char xch[PS ? 2 * XPAR + NW * 16 * 4 : 16];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, lg = lane >> 4;
@@ -231,8 +233,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
     // b = ii % NI of half hh = ii / NI; lane l reads chunk l % CPR of stage row
     // r = 16hh + b + NI*(l / CPR).  V likewise.  Interior stages add the lane's byte offset
     // to a wave-uniform base; the last, partial stage clamps each row to the range.
-    constexpr int KPW = 2 * R::NI / kWaves;  // DMA instructions per wave per tensor per stage
-    static_assert(KPW * kWaves == 2 * R::NI, "whole DMA blocks per wave");
+    constexpr int KPW = 2 * R::NI / NW;  // DMA instructions per wave per tensor per stage
+    static_assert(KPW * NW == 2 * R::NI, "whole DMA blocks per wave");
     const uint16_t *kvb = p.k + (size_t) kvh * p.kv_hs;
     const uint16_t *vvb = p.v + (size_t) kvh * p.kv_hs;
     const int nst = (j1 - j0 + kStageKeys - 1) / kStageKeys;
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
     // a flat one, whose wait also drains the ring's DMAs.)
     using lds_flag = __attribute__((address_space(3))) volatile unsigned;
     if constexpr (PS) {
-        if (lane < 2) *(lds_flag *) (xch + lane * XPAR + kWaves * XP + wave * 4) = 0u;
+        if (lane < 2) *(lds_flag *) (xch + lane * XPAR + NW * XP + wave * 4) = 0u;
     }
     // Positions of the tile's first and last rows (the host keeps positions below 2^31).
     const int qa_min = p.q_pos0 + (int) position_of((long long) tile * QT, p.G);
@@ -438,7 +440,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
             *reinterpret_cast<bf16x8 *>(xs + wave * XP + lane * 16) = pb[0];
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (lane == 0)
-                *(lds_flag *) (xs + kWaves * XP + wave * 4) = 2u * (unsigned) (s + 1) + (resc ? 1u : 0u);
+                *(lds_flag *) (xs + NW * XP + wave * 4) = 2u * (unsigned) (s + 1) + (resc ? 1u : 0u);
         }
 
         // O^T += V^T . P^T: lane (li, lg) gets dim 16dt + li of keys 4lg .. 4lg+3 (first
@@ -464,7 +466,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void prefill_kernel(PrefillParams p
             // The partner's flag for this stage (bounded: a wave that gave up would compute
             // garbage, not hang), then its P^T and, after its rescale, its factors.
             const unsigned want = 2u * (unsigned) (s + 1);
-            lds_flag *fl = (lds_flag *) (xs + kWaves * XP + (wave ^ 1) * 4);
+            lds_flag *fl = (lds_flag *) (xs + NW * XP + (wave ^ 1) * 4);
             unsigned f = __builtin_amdgcn_readfirstlane(*fl);
             for (int it = 0; (f & ~1u) != want && it < kPairSpin; ++it) {
                 __builtin_amdgcn_s_sleep(1);
@@ -860,16 +862,20 @@ bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u
 // over 1 .. 470 stages and 4 .. 512 workgroups; the plans then lie within 5% of the best
 // forced split on 40 of 45 random chunks (the others within 14%).
 struct Tiling {
-    int qb, kh;
+    int qb, kh, nw;
     float wg, stage;
-    int rows() const { return 16 * qb * (kh ? kWaves / 2 : kWaves); }
+    int rows() const { return 16 * qb * (kh ? nw / 2 : nw); }
 };
 
 // The forms a head dim can run.  At D = 256, per 32 keys: 64-row stage-halves tiles 0.66 us,
-// 128-row tiles 1.16, and 256-row tiles, whose two blocks share each K and V read, 1.9.
-constexpr Tiling kTilings512[] = {{1, 0, 9.0f, 1.5f}};
-constexpr Tiling kTilings256[] = {{1, 1, 5.5f, 0.66f}, {1, 0, 5.5f, 1.16f}, {2, 0, 8.0f, 1.9f}};
-constexpr Tiling kTilings128[] = {{2, 0, 3.5f, 1.0f}};
+// 128-row tiles 1.16, and 256-row tiles, whose two blocks share each K and V read, 1.9.  At D =
+// 512 a stage is bound by each wave's own chain, so four waves on 64 rows take nearly as long
+// as eight on 128; but where CUs would idle, the smaller tiles halve what each loads and
+// writes: 32 fresh tokens 15.9 -> 10.1 us, 100 18.6 -> 13.0, 16 over 5016 keys 32.4 -> 28.7, 20 over
+// 973 separate K / V rows 24.5 -> 21.3.
+constexpr Tiling kTilings512[] = {{1, 0, 4, 5.5f, 1.38f}, {1, 0, 8, 9.0f, 1.5f}};
+constexpr Tiling kTilings256[] = {{1, 1, 8, 5.5f, 0.66f}, {1, 0, 8, 5.5f, 1.16f}, {2, 0, 8, 8.0f, 1.9f}};
+constexpr Tiling kTilings128[] = {{2, 0, 8, 3.5f, 1.0f}};
 
 // Estimated us of a plan: `pieces(f)` calls f(stages) for each workgroup of one kv head in
 // dispatch order.  The heads run side by side, so one head has kTargetGroups / Hkv CUs; the
@@ -948,7 +954,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
     // unsplit and 80 us split in two.
     const long long rows = (long long) d->seq_q * p->G;
     const Tiling *forms = D == 512 ? kTilings512 : D == 256 ? kTilings256 : kTilings128;
-    const int nforms = D == 256 ? 3 : 1;
+    const int nforms = D == 512 ? 2 : D == 256 ? 3 : 1;
     float best = INFINITY;
     int kps = 0, most_stages = 0;  // of the best plan
     for (int f = 0; f < nforms; ++f) {
@@ -974,7 +980,10 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         auto consider = [&](int per) {  // per: stages per split
             const int splits = (most + per - 1) / per;
             float us = splits > 1 ? split_cost(4.0f * D * (float) rows * d->num_kv_heads * splits) : 0.0f;
-            if (us + t.wg + std::min(per, most) * t.stage >= best) return splits;
+            // no plan is faster than its longest workgroup, nor than its work spread evenly
+            if (us + std::max(t.wg + std::min(per, most) * t.stage,
+                              (float) (total * d->num_kv_heads / kTargetGroups)) >= best)
+                return splits;
             if (few && tiles * splits <= 2LL * kMaxRounds * kTargetGroups)
                 us += makespan(d->num_kv_heads, t, [&](auto &&piece) {
                     for (int i = 0; i < (int) tiles; ++i)
@@ -988,6 +997,7 @@ int plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
                 most_stages = most;
                 p->qb = t.qb;
                 p->kh = t.kh;
+                p->nw = t.nw;
                 p->tiles = (int) tiles;
             }
             return splits;
@@ -1019,9 +1029,11 @@ size_t workspace_of(const PrefillParams &p, int D) {
 template <int D>
 void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
     if (stages & 1) {
-        const dim3 grid(p.tiles * p.Hkv * p.splits), block(64 * kWaves);
+        const dim3 grid(p.tiles * p.Hkv * p.splits), block(64 * p.nw);
         if constexpr (D == 512) {
-            if (p.k == p.v) hipLaunchKernelGGL((prefill_kernel<512, 1, false, true, true, true>), grid, block, 0, st, p);
+            if (p.nw == 4 && p.k == p.v) hipLaunchKernelGGL((prefill_kernel<512, 1, false, true, true, true, 4>), grid, block, 0, st, p);
+            else if (p.nw == 4) hipLaunchKernelGGL((prefill_kernel<512, 1, false, false, false, false, 4>), grid, block, 0, st, p);
+            else if (p.k == p.v) hipLaunchKernelGGL((prefill_kernel<512, 1, false, true, true, true>), grid, block, 0, st, p);
             else hipLaunchKernelGGL((prefill_kernel<512, 1>), grid, block, 0, st, p);
         }
         else if constexpr (D == 128)

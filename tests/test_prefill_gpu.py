@@ -140,10 +140,23 @@ def test_split_merge_counts(D, Hq, Hkv, Sq, Sk, split_keys):
                 seed=31 + D)
 
 
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("Sq,past", [(64, 448), (600, 424)])
+def test_late_peaks_in_both_tile_heights_at_512(Sq, past, shared):
+    """Mid-stream rescales (as the test above) at the plan's two tile heights of head dim 512: 64
+    queries run four waves on 64-row tiles, 600 eight on 128-row tiles."""
+    Sk = past + Sq
+    peaks = [(h, i, past + i - d) for h, i, d in ((0, 5, 3), (3, 33, 17), (9, 60, 59), (17, Sq - 1, 1), (31, Sq - 2, 40))]
+    rows = sorted({0, 5, 33, 60, 63, Sq - 2, Sq - 1})
+    run_prefill(f"peaks-{Sq}-{int(shared)}", Hq=32, Hkv=4, D=512, Sq=Sq, Sk=Sk, q_pos0=past, k_pos0=0, seed=43,
+                shared=shared, peaks=peaks, rows=rows)
+
+
 @pytest.mark.parametrize("D,Hq,Hkv,Sq,past,window", [
     (512, 32, 4, 257, 700, 0),     # 17 tiles a head, the last of 8 rows: three splits fill one round
     (512, 16, 2, 16, 4900, 0),     # one full tile a head: tens of splits
     (512, 8, 8, 129, 0, 0),        # fresh, a last tile of one row
+    (512, 2, 1, 33, 3000, 0),      # two 64-row tiles, the last of two rows, many splits
     (256, 32, 16, 1100, 0, 256),   # 128-row tiles just past one round of the CUs
     (256, 16, 8, 17, 2000, 1024),  # short chunk: stage halves and splits together
     (256, 16, 8, 2470, 0, 1024),   # 128-row tiles in two uneven rounds
