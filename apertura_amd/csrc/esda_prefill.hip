@@ -698,8 +698,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 // lane), so a wave holds 64/LPR consecutive rows, and it does HG kv heads of them: their
 // loads are in flight together and share one set of cos / sin and k-norm weights.  4 heads
 // x 8256 rows 20.0 us (5.1 TB/s), x 16384 rows 33.5 (6.0); one wave per row with 8-byte
-// accesses, its own cos / sin and its own weight loads took 33.1 and 58.1.  The sum of squares is an fp32 sum over the row's lanes; rinv =
-// 1 / sqrt(mean + eps) with IEEE division and square root.
+// accesses, its own cos / sin and its own weight loads took 33.1 and 58.1.  The sum of squares is an
+// fp32 sum by pairs, within the lane and then over the row's lanes (a lane's 16 one after the
+// other leave it 3% further from the 64-bit sum); rinv = 1 / sqrt(mean + eps) with
+// IEEE division and square root.
 struct RawKvParams {
     const uint16_t *raw;        // bf16 rows, or NULL with q8 / scale / bias
     const unsigned char *q8;
@@ -773,11 +775,14 @@ __global__ __launch_bounds__(256) void raw_prefill_kv_kernel(RawKvParams p) {
                     x[half][e] = bf(raw[g][half], e);
                 }
             }
-        float ss = 0.0f;
+        float sq[8];
 #pragma unroll
-        for (int half = 0; half < 2; ++half)
+        for (int e = 0; e < 8; ++e) sq[e] = x[0][e] * x[0][e] + x[1][e] * x[1][e];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += x[half][e] * x[half][e];
+        for (int o = 4; o >= 1; o >>= 1)
+#pragma unroll
+            for (int e = 0; e < o; ++e) sq[e] += sq[e + o];
+        float ss = sq[0];
 #pragma unroll
         for (int o = LPR / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
         const float rinv = 1.0f / sqrtf(ss / (float) D + p.eps);
