@@ -983,10 +983,13 @@ void raw_attend_kernel(AttendParams p) {
                     const float rinv = __builtin_amdgcn_rsqf(ms);
                     rq = scl * rinv;
                     fq = bias * rinv;
+                    // Without a table both quotients are IEEE divisions: within half an ulp each, where
+                    // the reciprocal instruction is within one (~25 more VALU instructions a stage
+                    // beside the ~430 of the cos / sin).
                     if (lg == 0) {
                         xfw[0 * 16 + li] = rq;
-                        xfw[1 * 16 + li] = __builtin_amdgcn_rcpf(rq);
-                        xfw[2 * 16 + li] = bias * __builtin_amdgcn_rcpf(scl);
+                        xfw[1 * 16 + li] = TABLE ? __builtin_amdgcn_rcpf(rq) : 1.0f / rq;
+                        xfw[2 * 16 + li] = TABLE ? bias * __builtin_amdgcn_rcpf(scl) : bias / scl;
                     }
                 } else {
                     f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};

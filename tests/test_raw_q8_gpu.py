@@ -223,3 +223,33 @@ def test_q8_table_and_own_sincos_kernels_agree():
             assert err.max() <= TOL_MAX and err.mean() <= TOL_MEAN
     d = np.abs(o[1] - o[0])
     assert d.max() <= TOL_MAX and d.mean() <= TOL_MEAN
+
+
+def test_q8_own_sincos_centred_codes_give_exact_zeros():
+    """Rows whose bias is exactly -128 scales: bias / scale is -128 to the bit when it is a
+    division, so code 128 stands for exactly 0 and one visible row gives exactly 0 there (P * 128
+    and P * -128 cancel without rounding).  A quotient one ulp off leaves 2^-16 of the row's
+    scale instead.  256 single-row sequences of random scales (without a table)."""
+    from apertura_amd.decode import decode_raw_q8, new_raw_workspace, q8_step_for
+    rng = np.random.default_rng(71)
+    B, Hkv, cap = 64, 4, 16
+    qc = rng.integers(0, 256, (B, Hkv, cap, 512), dtype=np.uint8)
+    qc[..., ::2] = 128
+    sc = (0.002 + 0.05 * rng.random((B, Hkv, cap))).astype(np.float32)
+    bs = (-128.0 * sc).astype(np.float32)
+    q = orc.rms_norm_rows(orc.to_bf16(rng.standard_normal((B, Hkv, 512), dtype=np.float32)), None, 1e-6)
+    kw = orc.to_bf16((1.0 + 0.25 * rng.standard_normal(512)).astype(np.float32))
+    q8_d = torch.from_numpy(qc).cuda()
+    step = q8_step_for(q8_d, Hkv, eps=EPS, scale=512 ** -0.5)
+    out = decode_raw_q8(step, _dev(q), None, q8_d, torch.from_numpy(sc).cuda(), torch.from_numpy(bs).cuda(),
+                        torch.zeros(B, dtype=torch.int32, device="cuda"), _dev(kw),
+                        torch.from_numpy(orc.rope_inv_freq(512, 1.0e6, 0.25)).cuda(),
+                        workspace=new_raw_workspace(step, "cuda"))
+    torch.cuda.synchronize()
+    o = orc.from_bf16(_host(out)).reshape(B, Hkv, 512).astype(np.float64)
+    bad = int((o[..., ::2] != 0).any(-1).sum())
+    print(f"[q8] centred codes: {bad} of {B * Hkv} rows are not exactly 0 at code 128", flush=True)
+    assert bad == 0
+    x = qc[:, :, 0].astype(np.float64) * sc[:, :, :1] + bs[:, :, :1]
+    ref = x / np.sqrt((x * x).mean(-1, keepdims=True) + EPS)
+    assert np.abs(o - ref).max() <= TOL_MAX
