@@ -992,18 +992,39 @@ void raw_attend_kernel(AttendParams p) {
                         xfw[2 * 16 + li] = TABLE ? bias * __builtin_amdgcn_rcpf(scl) : bias / scl;
                     }
                 } else {
-                    f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int kk = 0; kk < 16; ++kk) {
-                        xr[kk] = *reinterpret_cast<const u32x4 *>(sl + li * kBlk + 2 * kdim(kk, lg));
-                        const bf16x8 x = __builtin_bit_cast(bf16x8, xr[kk]);
-                        g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, x, g, 0, 0, 0);
-                    }
-                    // Row factors (C layout: lane (li, lg) holds C[4lg + i][li]; row li's diagonal
-                    // is register li - 4lg of the lanes with lg == li / 4, which publish them).
+                    // C layout: lane (li, lg) holds C[4lg + i][li]; row li's diagonal is register
+                    // li - 4lg of the lanes with lg == li / 4, which publish the row factors.
                     const int i = li - 4 * lg;
+                    auto diagonal = [&](const f32x4 &g) { return i == 0 ? g[0] : i == 1 ? g[1] : i == 2 ? g[2] : g[3]; };
+                    f32x4 g = {0.0f, 0.0f, 0.0f, 0.0f};
+                    float sq[8];
+                    if constexpr (TABLE) {
+#pragma unroll
+                        for (int kk = 0; kk < 16; ++kk) {
+                            xr[kk] = *reinterpret_cast<const u32x4 *>(sl + li * kBlk + 2 * kdim(kk, lg));
+                            const bf16x8 x = __builtin_bit_cast(bf16x8, xr[kk]);
+                            g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, x, g, 0, 0, 0);
+                        }
+                    } else {
+                        // Eight chains of two k-steps, added by pairs: a chain of sixteen drops every
+                        // 32-dim sum below half an ulp of the running one (and each diagonal is taken
+                        // at once: eight live accumulators do not fit beside O^T and Q^T).
+#pragma unroll
+                        for (int kk = 0; kk < 16; ++kk) xr[kk] = *reinterpret_cast<const u32x4 *>(sl + li * kBlk + 2 * kdim(kk, lg));
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) {
+                            const bf16x8 x0 = __builtin_bit_cast(bf16x8, xr[c]), x1 = __builtin_bit_cast(bf16x8, xr[c + 8]);
+                            const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+                            sq[c] = diagonal(__builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                x1, x1, __builtin_amdgcn_mfma_f32_16x16x32_bf16(x0, x0, z, 0, 0, 0), 0, 0, 0));
+                        }
+#pragma unroll
+                        for (int o = 4; o >= 1; o >>= 1)
+#pragma unroll
+                            for (int c = 0; c < o; ++c) sq[c] += sq[c + o];
+                    }
                     if (i >= 0 && i < 4) {
-                        const float s2 = i == 0 ? g[0] : i == 1 ? g[1] : i == 2 ? g[2] : g[3];
+                        const float s2 = TABLE ? diagonal(g) : sq[0];
                         const float ms = s2 * (1.0f / kRawDim) + p.eps;
                         const float rinv = __builtin_amdgcn_rsqf(ms);
                         xfw[0 * 16 + li] = rinv;

@@ -319,3 +319,35 @@ def test_es_decode_attn_global_over_more_streams_than_scratch_sets():
     assert all(np.array_equal(_host(o), first) for o in outs[1:])
     _check_conditioned("12 streams", orc.from_bf16(_host(outs[-1])).reshape(8 * Hkv, 512).astype(np.float64), q[0],
                        np.ascontiguousarray(raw[0]), length, kw, np.asarray(inv, np.float32), 1.0)
+
+
+def test_raw_own_sincos_row_norms_of_one_large_element():
+    """One element of 2^12 or more beside 511 of about 0.15: in a chain of sixteen 32-dim partial
+    sums every one after the first is below half an ulp of the sum and is lost (6e-7 of the
+    norm's square), in four chains of four only the first chain's three are.  One visible row
+    gives V = x * rinv, so the lost part shows as elements on the wrong side of a bf16 rounding
+    boundary: by the share of boundaries within the error, about 62 of the 1,046,528 elements
+    against 18 (rounding of rinv, 1 / rinv and the quotient: 8e-8 on average)."""
+    from apertura_amd.decode import RawStep, decode_raw, new_raw_workspace
+    rng = np.random.default_rng(73)
+    B, Hkv, cap = 256, 8, 16
+    x = (0.12 + 0.056 * rng.random((B, Hkv, cap, 512), dtype=np.float32)) * rng.choice([-1.0, 1.0], (B, Hkv, cap, 512))
+    x[..., 0] = 4100.0 + 600.0 * rng.random((B, Hkv, cap))
+    x[..., 1:8] = 1000.0 * rng.random((B, Hkv, cap, 7))  # (beside it in the first partial sum: many norms)
+    raw = orc.to_bf16(x.astype(np.float32))
+    q = orc.to_bf16(rng.standard_normal((B, Hkv, 512), dtype=np.float32))
+    kw = orc.to_bf16(np.ones(512, dtype=np.float32))
+    step = RawStep(batch=B, num_q_heads=Hkv, num_kv_heads=Hkv, cap=cap, eps=EPS, scale=512 ** -0.5)
+    out = decode_raw(step, _dev(q), None, _dev(raw), torch.zeros(B, dtype=torch.int32, device="cuda"), _dev(kw),
+                     torch.from_numpy(orc.rope_inv_freq(512, 1.0e6, 0.25)).cuda(),
+                     workspace=new_raw_workspace(step, "cuda"))
+    torch.cuda.synchronize()
+    r = orc.from_bf16(raw[:, :, 0]).astype(np.float64)
+    ref = r / np.sqrt((r * r).mean(-1, keepdims=True) + EPS)
+    m, e = np.frexp(ref)  # bf16 keeps 8 significant bits: m * 256 rounded (half to even)
+    want = np.ldexp(np.rint(m * 256.0), e - 8)
+    got = orc.from_bf16(_host(out)).reshape(B, Hkv, 512).astype(np.float64)
+    assert np.abs(got - ref).max() <= TOL_MAX * np.abs(ref).max()
+    off = int((got[..., 8:] != want[..., 8:]).sum())
+    print(f"[raw] {off} of {want[..., 8:].size} elements differ from the correctly rounded 64-bit rows", flush=True)
+    assert off <= 36
