@@ -141,8 +141,9 @@ constexpr int kRopePairs = 64;
 // sequence) rows [split * chunk, ...) of its pair; balanced plans give workgroup w its share
 // of all visible rows of the batch, walked pair by pair (esda_plan.h).  segment(b, kvh, j0,
 // j1, view, slot, direct) runs each; the ring is free again when it returns (the walk puts
-// a barrier between segments).  NW: waves per workgroup.
-template <int NW, class Seg>
+// a barrier between segments).  NW: waves per workgroup; PAD: rows a pair counts beside its
+// own in a balanced plan's shares.
+template <int NW, int PAD = 0, class Seg>
 __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segment) {
     const int wg = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -177,7 +178,7 @@ __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segme
     if (single) {
         // one sequence: its view straight from the (wave-uniform) position word
         w_view = seq_view(p.pos[0], p.row_base ? p.row_base[0] : 0, p.cap, p.window, p.ring);
-        rows_seq = w_view.ok ? w_view.nvis : 0;
+        rows_seq = w_view.ok ? w_view.nvis + PAD : 0;
         if (wg == 0 && tid == 0) {
             if (!w_view.ok) atomicAdd(p.status, 1);
             esda_plan::write_prefix_entry(p.table, 0, 1, 0, rows_seq);
@@ -186,7 +187,7 @@ __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segme
         const int t = wave_scan ? lane : tid;
         SeqView v{0, 0, 0, 0};
         if (t < p.B) v = seq_view(p.pos[t], p.row_base ? p.row_base[t] : 0, p.cap, p.window, p.ring);
-        const long long nv = v.ok ? v.nvis : 0;
+        const long long nv = v.ok ? v.nvis + PAD : 0;
         long long x = nv;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -266,10 +267,13 @@ __device__ __forceinline__ void walk_segments(const AttendParams &p, Seg &&segme
         // Every value of the segment is the same in all lanes (computed from LDS and kernel
         // arguments); saying so keeps the ring's control flow and addresses scalar.
         const SeqView sv{uniform(v.nvis), uniform(v.first), uniform(v.newrow), uniform(v.ok)};
-        const int ub = uniform(b), ukvh = uniform(kvh), uj0 = uniform(j0), uj1 = uniform(j1);
-        segment(ub, ukvh, uj0, uj1, sv, (size_t) esda_plan::share_slot((long long) ub * p.Hkv + ukvh, wg),
-                uj0 == 0 && uj1 == n);
-        lds_barrier();  // every wave is done with the ring before the next segment refills it
+        const int ub = uniform(b), ukvh = uniform(kvh), uj0 = uniform(j0);
+        const int uj1 = PAD ? min(uniform(j1), sv.nvis) : uniform(j1), un = PAD ? sv.nvis : n;
+        if (PAD == 0 || uj0 < un) {
+            segment(ub, ukvh, uj0, uj1, sv, (size_t) esda_plan::share_slot((long long) ub * p.Hkv + ukvh, wg),
+                    uj0 == 0 && uj1 == un);
+            lds_barrier();  // every wave is done with the ring before the next segment refills it
+        }
         x = seg_end;
     }
 }
@@ -641,6 +645,14 @@ __device__ __forceinline__ constexpr bool rot_step(int kk) { return (kk & 7) < 2
 // with the generic threshold of 8 about half of all stages would rescale.
 constexpr float kRawRescaleSlack = 64.0f;
 
+// Balanced shares without a table: a pair counts this many rows beside its own, about what
+// starting its segment costs (~6 us: q, the first rows, the waves' merge, each a round trip;
+// a row of a long segment takes 0.05), so that no share collects many short pairs.  8 heads x
+// 61, 4 and 101 rows 59.2 us a step with 0 and 18.1 with 128 (the tiny sequence's 8 segments
+// were one share), 15.4 with 64, 17.6 with 256; 3 x 129 rows 21.5, 18.2, 21.2, 21.0; 16
+// sequences of 6 .. 156 rows 54.4, 20.3, 22.9, 22.0; 7 x 1030 x 4 heads 28.2, 22.2, 24.8, 24.1.
+constexpr int kOwnTablePad = 128;
+
 template <bool Q8, bool TABLE>
 struct WRing {
     static constexpr int ROWS = Q8 ? 8 * kBlk : 16 * kBlk;  // a stage's 16 rows (q8: two per block)
@@ -681,17 +693,19 @@ void raw_attend_kernel(AttendParams p) {
     // q8: the k-norm weights in fp32, read per k-step (the lanes of a lane group read the
     // same 32 bytes); 128 of them per lane would not fit in registers beside O^T and Q^T.
     __shared__ __attribute__((aligned(16))) float kwl[Q8 ? kRawDim : 1];
-    // no table: the rotary frequencies, read back per stage
-    __shared__ __attribute__((aligned(16))) float invl[TABLE ? 1 : kRopePairs];
-    if constexpr (!TABLE) {
-        if (tid < kRopePairs) invl[tid] = p.inv_freq[tid];
-    }
+    // no table: the rotary frequencies, a copy per wave (no barrier), read back per stage.  A call
+    // of a few stages is latency from end to end: with the copy ahead of every DMA, the first
+    // rows requested before q and the cos / sin computed while they are in flight, 31 rows x 4
+    // heads take 9.0 us against 9.7 (q8 10.4 against 11.7).
+    __shared__ __attribute__((aligned(16))) float invl[TABLE ? 1 : kWaves][kRopePairs];
+    float freq = 0.0f;
+    if constexpr (!TABLE) freq = p.inv_freq[lane];
     if constexpr (Q8) {
         const unsigned t = reinterpret_cast<const unsigned *>(p.kw)[tid];
         kwl[2 * tid] = bf16_lo(t);
         kwl[2 * tid + 1] = bf16_hi(t);
     }
-    if constexpr (Q8 || !TABLE) __syncthreads();
+    if constexpr (Q8) __syncthreads();
     // Raw: the A operands of the x * kw products, diag(kw) over 16 dims.  For k-step kk and half
     // hh the B operand is the lane's own dims kdim(kk, lg) + 4hh .. + 3 of row li; lane
     // (li, lg) then holds kw of dim kdim(kk, lg) + 4hh + (li & 3) at slot li & 3 when
@@ -712,6 +726,9 @@ void raw_attend_kernel(AttendParams p) {
         }
     }
 
+    // (ahead of any DMA: a wait for this load must not wait for rows behind it)
+    if constexpr (!TABLE) invl[wave][lane] = freq;
+
     auto segment = [&](const int b, const int kvh, const int j0, const int j1, const SeqView sv, const size_t slot,
                        const bool direct) {
         const bool append = p.k_new != nullptr;
@@ -723,7 +740,7 @@ void raw_attend_kernel(AttendParams p) {
 
         // Q^T operand: head li of the packed pair (zero for padding heads li >= G)
         bf16x8 qv[16];
-        {
+        auto load_q = [&]() {
             const bool qok = li < p.G;
             const uint16_t *qrow = p.q + ((size_t) b * p.Hq + (size_t) kvh * p.G + (qok ? li : 0)) * kRawDim;
 #pragma unroll
@@ -731,7 +748,8 @@ void raw_attend_kernel(AttendParams p) {
                 const u32x4 t = qok ? *reinterpret_cast<const u32x4 *>(qrow + kdim(kk, lg)) : u32x4{0u, 0u, 0u, 0u};
                 qv[kk] = __builtin_bit_cast(bf16x8, t);
             }
-        }
+        };
+        if constexpr (TABLE) load_q();
         if constexpr (Q8) {
             // The new row is quantized into the cache before any DMA (wave 0),
             // esQuantizeRawRows' arithmetic (ESDecodeAttn.mm:491-509).
@@ -772,9 +790,12 @@ void raw_attend_kernel(AttendParams p) {
                 }
             }
         }
-        ESDA_WAIT_VM(0);  // operands in registers (and the q8 row stored) before the ring counts its loads
+        if constexpr (TABLE) ESDA_WAIT_VM(0);  // operands in registers (and the q8 row stored) before the ring counts its loads
         if constexpr (Q8) {
-            if (append && j1 == sv.nvis) lds_barrier();  // the quantized row is in memory before any DMA
+            if (append && j1 == sv.nvis) {
+                if constexpr (!TABLE) ESDA_WAIT_VM(0);
+                lds_barrier();  // the quantized row is in memory before any DMA
+            }
         }
 
         const int nst = (j1 - j0 + 15) >> 4;  // 16-row stages: 16 positions
@@ -878,6 +899,7 @@ void raw_attend_kernel(AttendParams p) {
             dma_rows(st0, wl);
             if constexpr (TABLE) dma_tab(st0);
         }
+        if constexpr (!TABLE) load_q();  // behind the first rows: one round trip for both
 
         float m = -INFINITY, l = 0.0f;
         float bt = 0.0f;  // q8: sum of P * bias / scale of this lane's head
@@ -888,6 +910,22 @@ void raw_attend_kernel(AttendParams p) {
 
         for (int st = st0, it = 0; st < nst; st += kWaves, ++it) {
             unsigned char *const sl = wl + (it & 1) * W::SLOT;
+            u32x4 tab[4];
+            if constexpr (!TABLE) {
+                // Computed (rope_table_kernel's arithmetic; the lanes of a stage need 16 x 64 pairs, so
+                // each computes the 16 it uses) while the stage's rows are in flight
+                const float t = (float) (sv.first + min(j0 + 16 * st + li, j1 - 1));
+#pragma unroll
+                for (int c4 = 0; c4 < 4; ++c4) {
+                    const f32x4 f = *reinterpret_cast<const f32x4 *>(&invl[wave][32 * (c4 >> 1) + 8 * lg + 4 * (c4 & 1)]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float sn, cs;
+                        sincos_f32(t * f[e], sn, cs);
+                        tab[c4][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{cs, sn}, bf16x2));
+                    }
+                }
+            }
             ESDA_WAIT_VM(0);  // this stage's rows and table rows landed
             unsigned char *const nsl = wl + ((it + 1) & 1) * W::SLOT;
             const bool more = st + kWaves < nst;
@@ -899,24 +937,8 @@ void raw_attend_kernel(AttendParams p) {
             // Scores S^T[16 rows x 16 heads] of K = bf16(rope(x * rinv * kw)) (q8: x = q * scale
             // + bias), rounded where ESDecodeAttn.mm:51-93 rounds it.
             f32x4 sp0 = {0.0f, 0.0f, 0.0f, 0.0f}, sp1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            // cos / sin of row li's position for the rotary pairs this lane holds: from the
-            // table, or computed (rope_table_kernel's arithmetic; the lanes of a stage need
-            // 16 x 64 pairs, so each computes the 16 it uses)
+            // cos / sin of row li's position for the rotary pairs this lane holds, from the table
             auto load_tab = [&](u32x4 (&tab)[4]) {
-                if constexpr (!TABLE) {
-                    const float t = (float) (sv.first + min(j0 + 16 * st + li, j1 - 1));
-#pragma unroll
-                    for (int c4 = 0; c4 < 4; ++c4) {
-                        const f32x4 f = *reinterpret_cast<const f32x4 *>(invl + 32 * (c4 >> 1) + 8 * lg + 4 * (c4 & 1));
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            float sn, cs;
-                            sincos_f32(t * f[e], sn, cs);
-                            tab[c4][e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{cs, sn}, bf16x2));
-                        }
-                    }
-                    return;
-                }
                 const int bt2 = li >> 2, rib = li & 3;  // row li: position li of the stage
 #pragma unroll
                 for (int c4 = 0; c4 < 4; ++c4) {
@@ -1045,8 +1067,7 @@ void raw_attend_kernel(AttendParams p) {
             // Other lanes read the factors back: a compiler memory barrier keeps those loads
             // after the stores above (the lanes' LDS accesses then run in order).
             asm volatile("" ::: "memory");
-            u32x4 tab[4];
-            load_tab(tab);
+            if constexpr (TABLE) load_tab(tab);
             const float rk = Q8 ? rq : xfw[0 * 16 + li];  // rinv of row li (q8: scale * rinv)
             // Pass 2: x * rinv * kw of k-step kk, dims kdim(kk, lg) .. + 7 of row li.
             auto xkw = [&](int kk, float (&v)[8]) {
@@ -1232,7 +1253,7 @@ void raw_attend_kernel(AttendParams p) {
         }
         lds_barrier();  // the merge area is read before the next segment's DMA overwrites it
     };
-    walk_segments<kWaves>(p, segment);
+    walk_segments<kWaves, TABLE ? 0 : kOwnTablePad>(p, segment);
 }
 
 struct MergeParams {
@@ -1242,6 +1263,7 @@ struct MergeParams {
     uint16_t *out;
     int B, Hq, Hkv, G, D, cap, window, ring;
     int balanced, W, S, chunk;
+    int pad;  // balanced: rows a pair counted beside its own (walk_segments' PAD)
 };
 
 constexpr int kMergeThreads = 256;
@@ -1267,7 +1289,7 @@ __device__ __forceinline__ int pair_splits(const MergeParams &p, int b, int kvh,
         // The attend workgroups w0 .. w1 that covered pair (b, kvh) (every one of them holds
         // rows of the pair and wrote its slot); an inconsistent table reads nothing.
         int w0 = 0;
-        ns = esda_plan::pair_owners(p.table[b], p.table[b + 1], p.table[p.B], p.Hkv, kvh, p.W, &w0);
+        ns = esda_plan::pair_owners(p.table[b], p.table[b + 1], p.table[p.B], p.Hkv, kvh, p.W, &w0, p.pad);
         if (ns == 0) return 0;
         pbase = (size_t) esda_plan::share_slot((long long) b * p.Hkv + kvh, w0);
     } else {
@@ -1818,6 +1840,7 @@ int run_stages(const esda_decode_desc *d, const Plan &pl, const AttendParams &ap
         mp.W = pl.W;
         mp.S = pl.S;
         mp.chunk = pl.chunk;
+        mp.pad = mode != 0 && !ap_in.rope_tab ? kOwnTablePad : 0;
         // Partials per pair: a grid's S, or about W / pairs + 1 of the balanced shares.
         const long long pairs = (long long) d->batch * d->num_kv_heads / pl.pk;
         if (pl.balanced ? pl.W < kMergeShares * pairs : pl.S <= kMergeRowsChunk) {

@@ -112,13 +112,15 @@ ESDA_HD long long share_slot(long long u, int w) { return u + w; }
 // The workgroups w0 .. w1 whose shares hold rows of pair (b, kvh) -- those holding its
 // first and last rows -- for the merge, from the prefix table entries table_b = table[b],
 // table_b1 = table[b + 1] and table_total = table[B].  Returns their count (0 for a
-// sequence with no rows or an inconsistent table) and sets *w0.
+// sequence with no rows or an inconsistent table) and sets *w0.  pad: rows every pair of a
+// sequence with rows counted in the table beside its own, after them (nobody's work: they
+// only move the shares' ends).
 ESDA_HD int pair_owners(long long table_b, long long table_b1, long long table_total, int Hkv, int kvh, int W,
-                        int *w0) {
+                        int *w0, int pad = 0) {
     const long long n = table_b1 - table_b;
     const long long rows_total = table_total * Hkv;
-    if (n <= 0 || rows_total <= 0) return 0;
-    const long long first = table_b * Hkv + (long long) kvh * n, last = first + n - 1;
+    if (n <= pad || rows_total <= 0) return 0;
+    const long long first = table_b * Hkv + (long long) kvh * n, last = first + n - pad - 1;
     if (first < 0 || last >= rows_total) return 0;
     const long long Wr = rows_total < W ? rows_total : W;
     // workgroup w holds row r iff share_begin(w) <= r < share_begin(w + 1), i.e. the

@@ -10,6 +10,9 @@
 // non-empty; the segments of a pair cover its rows exactly once, in order; the merge's
 // owners w0 .. w1 are exactly the workgroups that wrote the pair's slots, and those slots
 // are distinct across pairs; a pair covered by one workgroup is the one written directly.
+// Half of the batches count `pad` rows beside each pair's own, as the raw kernels' plans
+// without a rotary table do: then no share starts more than its length / (pad + 1) + 2
+// segments, however short the sequences.
 // Grid splits: the splits of a pair cover [0, nvis) exactly once and the merge's count
 // matches.  PLANT_TABLE_BUG: the prefix table's total is written by thread B (which a
 // 256-sequence batch does not have) -- the checker must report it.
@@ -38,7 +41,7 @@ static int g_fail = 0;
     } while (0)
 
 struct Batch {
-    int B, Hkv, W, cap, window, ring;
+    int B, Hkv, W, cap, window, ring, pad;
     std::vector<int> pos, base;
 };
 
@@ -65,7 +68,7 @@ static void check_balanced(const Batch &bt) {
     long long rows_seq = 0;
     for (int b = 0; b < B; ++b) {
         const SeqView v = seq_view(bt.pos[b], bt.base[b], bt.cap, bt.window, bt.ring);
-        nv[b] = v.ok ? v.nvis : 0;
+        nv[b] = v.ok ? v.nvis + bt.pad : 0;
         rows_seq += nv[b];
     }
     const int threads = B <= 64 ? 64 : 256;  // the wave scan, or the workgroup's LDS scan
@@ -84,7 +87,7 @@ static void check_balanced(const Batch &bt) {
         const long long lo = share_begin(rows_total, Wr, w), hi = share_begin(rows_total, Wr, w + 1);
         CHECK(lo < hi, "B=%d W=%d: share %d empty [%lld, %lld)", B, bt.W, w, lo, hi);
         long long x = lo;
-        int guard = 0;
+        int guard = 0, started = 0;
         while (x < hi && ++guard < 100000) {
             // the kernel's rule: b = the number of sequences whose rows end at or before x
             int b = 0;
@@ -96,10 +99,16 @@ static void check_balanced(const Batch &bt) {
             CHECK(sg.kvh >= 0 && sg.kvh < Hkv && sg.j0 >= 0 && sg.j1 <= n && sg.j0 < sg.j1,
                   "bad segment kvh=%d j0=%d j1=%d n=%d", sg.kvh, sg.j0, sg.j1, n);
             const long long u = (long long) b * Hkv + sg.kvh;
-            segs[u].push_back({sg.j0, sg.j1, w, share_slot(u, w), sg.j0 == 0 && sg.j1 == n});
+            const int nr = n - bt.pad, j1 = std::min(sg.j1, nr);
+            if (sg.j0 < nr) {
+                segs[u].push_back({sg.j0, j1, w, share_slot(u, w), sg.j0 == 0 && j1 == nr});
+                ++started;
+            }
             CHECK(sg.end > x, "no progress");
             x = sg.end;
         }
+        CHECK(started <= (hi - lo) / (bt.pad + 1) + 2, "W=%d pad=%d: share %d of %lld rows starts %d segments", bt.W,
+              bt.pad, w, hi - lo, started);
     }
     std::vector<char> slot_used((size_t) B * Hkv + bt.W, 0);
     for (int b = 0; b < B; ++b)
@@ -116,9 +125,10 @@ static void check_balanced(const Batch &bt) {
                     slot_used[g.slot] = 1;
                 }
             }
-            CHECK(at == nv[b], "pair (%d,%d): covered %d of %lld rows", b, h, at, nv[b]);
+            const long long rows = nv[b] ? nv[b] - bt.pad : 0;
+            CHECK(at == rows, "pair (%d,%d): covered %d of %lld rows", b, h, at, rows);
             int w0 = -1;
-            const int ns = pair_owners(table[b], table[b + 1], table[B], Hkv, h, bt.W, &w0);
+            const int ns = pair_owners(table[b], table[b + 1], table[B], Hkv, h, bt.W, &w0, bt.pad);
             CHECK(ns == (int) s.size(), "pair (%d,%d): merge reads %d splits, %zu written", b, h, ns, s.size());
             for (int i = 0; i < (int) s.size() && i < ns; ++i)
                 CHECK(s[i].w == w0 + i, "pair (%d,%d): owner %d is workgroup %d, merge expects %d", b, h, i, s[i].w,
@@ -157,6 +167,7 @@ int main(int argc, char **argv) {
         bt.B = limit ? 256 : (it % 5 == 0 ? U(65, 256) : U(1, 64));
         bt.Hkv = limit ? 16 : U(1, 16);
         bt.W = limit ? 16384 : (U(0, 3) == 0 ? U(1, 16384) : U(1, 512));
+        bt.pad = it % 2 ? 128 : 0;
         bt.ring = U(0, 3) == 0;
         bt.cap = limit ? U(1 << 16, 1 << 20) : U(1, 40000);
         bt.window = bt.ring ? U(1, bt.cap) : (U(0, 1) ? 0 : U(1, bt.cap));

@@ -351,3 +351,14 @@ def test_raw_own_sincos_row_norms_of_one_large_element():
     off = int((got[..., 8:] != want[..., 8:]).sum())
     print(f"[raw] {off} of {want[..., 8:].size} elements differ from the correctly rounded 64-bit rows", flush=True)
     assert off <= 36
+
+
+@pytest.mark.parametrize("B,Hkv,pos", [
+    (3, 8, [60, 3, 100]),                            # a share per head of the 4-row sequence, not all in one
+    (70, 2, [(37 * i) % 200 for i in range(70)]),    # the scan of more than 64 sequences; rows of 1 .. 200
+    (5, 1, [0, 0, 0, 0, 199]),                       # four single rows beside a long pair
+])
+def test_raw_own_sincos_shares_of_short_sequences(B, Hkv, pos):
+    """Without a table the shares of a balanced plan count a start-up cost per pair beside its
+    rows: segments, partials and the merge's owners of sequences far shorter than that cost."""
+    run_raw(f"short-{B}", B=B, Hq=8 * Hkv, Hkv=Hkv, cap=200, pos=pos, scale=512 ** -0.5, seed=80 + B)

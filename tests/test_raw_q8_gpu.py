@@ -253,3 +253,14 @@ def test_q8_own_sincos_centred_codes_give_exact_zeros():
     x = qc[:, :, 0].astype(np.float64) * sc[:, :, :1] + bs[:, :, :1]
     ref = x / np.sqrt((x * x).mean(-1, keepdims=True) + EPS)
     assert np.abs(o - ref).max() <= TOL_MAX
+
+
+@pytest.mark.parametrize("B,Hkv,pos", [
+    (3, 8, [60, 3, 100]),                            # a share per head of the 4-row sequence, not all in one
+    (70, 2, [(37 * i) % 200 for i in range(70)]),    # the scan of more than 64 sequences; rows of 1 .. 200
+    (5, 1, [0, 0, 0, 0, 199]),                       # four single rows beside a long pair
+])
+def test_q8_own_sincos_shares_of_short_sequences(B, Hkv, pos):
+    """Without a table the shares of a balanced plan count a start-up cost per pair beside its
+    rows: segments, partials and the merge's owners of sequences far shorter than that cost."""
+    run_q8(f"short-{B}", B=B, Hq=8 * Hkv, Hkv=Hkv, cap=200, pos=pos, scale=512 ** -0.5, seed=80 + B)
