@@ -23,7 +23,6 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 // Loads and stores of rows that need only their element's alignment.
 typedef unsigned u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef unsigned u32x2_a1 __attribute__((ext_vector_type(2), aligned(1)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 

@@ -693,10 +693,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 
 // ------------------------------------------------------------ raw-K reconstruction
 //
-// Memory-bound: a raw row read, a K and a V row written.  LPR = D/16 lanes hold a row, each
-// 8 dims of either half (16-byte loads and stores; every rotary pair (d, d + D/2) in one
+// Memory-bound: a raw row read, a K and a V row written.  LPR = D / 2E lanes hold a row, each
+// E dims of either half (E = 8: 16-byte loads and stores; every rotary pair (d, d + D/2) in one
 // lane), so a wave holds 64/LPR consecutive rows, and it does HG kv heads of them: their
-// loads are in flight together and share one set of cos / sin and k-norm weights.  4 heads
+// loads are in flight together and share one set of cos / sin and k-norm weights.  Few rows
+// take fewer dims a lane (launch_raw_kv).  4 heads
 // x 8256 rows 20.0 us (5.1 TB/s), x 16384 rows 33.5 (6.0); one wave per row with 8-byte
 // accesses, its own cos / sin and its own weight loads took 33.1 and 58.1.  The sum of squares is an
 // fp32 sum by pairs, within the lane and then over the row's lanes (a lane's 16 one after the
@@ -716,10 +717,13 @@ struct RawKvParams {
 
 __device__ __forceinline__ float bf16r(float x) { return (float) (__bf16) x; }
 
-template <int D, bool Q8, int HG>
+template <int D, bool Q8, int HG, int E>
 __global__ __launch_bounds__(256) void raw_prefill_kv_kernel(RawKvParams p) {
 #pragma clang fp contract(off)  // every rounding point as written (no fused multiply-add)
-    constexpr int HALF = D / 2, LPR = D / 16, RPW = 64 / LPR;
+    constexpr int HALF = D / 2, LPR = HALF / E, RPW = 64 / LPR;
+    typedef uint16_t row_piece __attribute__((ext_vector_type(E), aligned(2)));
+    typedef unsigned char code_piece __attribute__((ext_vector_type(E), aligned(1)));
+    typedef __bf16 out_piece __attribute__((ext_vector_type(E)));
     const int lane = threadIdx.x & 63, l = lane % LPR;
     const long long wv = (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
     const int row_groups = (p.rows + RPW - 1) / RPW;
@@ -728,80 +732,77 @@ __global__ __launch_bounds__(256) void raw_prefill_kv_kernel(RawKvParams p) {
     const int tt = (int) (wv % row_groups) * RPW + lane / LPR;
     const int t = min(tt, p.rows - 1);  // rows past the end repeat the last one, unwritten
 
-    u32x4 raw[HG][2];
+    row_piece raw[HG][2];
+    code_piece code[Q8 ? HG : 1][2];
     float sc[HG], bs[HG];
 #pragma unroll
     for (int g = 0; g < HG; ++g) {
         const int h = min(h0 + g, p.Hkv - 1);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-            const size_t at = (size_t) h * p.raw_hs + (size_t) t * D + half * HALF + 8 * l;
-            if constexpr (Q8) {
-                const u32x2 w = *reinterpret_cast<const u32x2_a1 *>(p.q8 + at);
-                raw[g][half] = u32x4{w[0], w[1], 0u, 0u};
-            } else {
-                raw[g][half] = *reinterpret_cast<const u32x4_a2 *>(p.raw + at);
-            }
+            const size_t at = (size_t) h * p.raw_hs + (size_t) t * D + half * HALF + E * l;
+            if constexpr (Q8) code[g][half] = *reinterpret_cast<const code_piece *>(p.q8 + at);
+            else raw[g][half] = *reinterpret_cast<const row_piece *>(p.raw + at);
         }
         if constexpr (Q8) {
             sc[g] = p.sc[(size_t) h * p.sb_hs + t];
             bs[g] = p.bs[(size_t) h * p.sb_hs + t];
         }
     }
-    const u32x4 kwa = *reinterpret_cast<const u32x4_a2 *>(p.kw + 8 * l);
-    const u32x4 kwb = *reinterpret_cast<const u32x4_a2 *>(p.kw + HALF + 8 * l);
-    auto bf = [](const u32x4 &w, int e) { return e & 1 ? bf16_hi(w[e / 2]) : bf16_lo(w[e / 2]); };
-    float c[8], s[8];
+    const row_piece kwa = *reinterpret_cast<const row_piece *>(p.kw + E * l);
+    const row_piece kwb = *reinterpret_cast<const row_piece *>(p.kw + HALF + E * l);
+    auto bf = [](uint16_t w) { return __builtin_bit_cast(float, (unsigned) w << 16); };
+    float c[E], s[E];
     const float pos = (float) (p.pos0 + t);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < E; ++e) {
         float sn, cs;
-        sincos_f32(pos * p.inv_freq[8 * l + e], sn, cs);
+        sincos_f32(pos * p.inv_freq[E * l + e], sn, cs);
         c[e] = bf16r(cs);
         s[e] = bf16r(sn);
     }
 #pragma unroll
     for (int g = 0; g < HG; ++g) {
         if (h0 + g >= p.Hkv) break;
-        float x[2][8];
+        float x[2][E];
 #pragma unroll
         for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            for (int e = 0; e < E; ++e) {
                 if constexpr (Q8) {
-                    const float prod = (float) ((raw[g][half][e / 4] >> (8 * (e % 4))) & 255u) * sc[g];
+                    const float prod = (float) code[g][half][e] * sc[g];
                     x[half][e] = bf16r(prod + bs[g]);  // the bf16 raw view of the q8 row
                 } else {
-                    x[half][e] = bf(raw[g][half], e);
+                    x[half][e] = bf(raw[g][half][e]);
                 }
             }
-        float sq[8];
+        float sq[E];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sq[e] = x[0][e] * x[0][e] + x[1][e] * x[1][e];
+        for (int e = 0; e < E; ++e) sq[e] = x[0][e] * x[0][e] + x[1][e] * x[1][e];
 #pragma unroll
-        for (int o = 4; o >= 1; o >>= 1)
+        for (int o = E / 2; o >= 1; o >>= 1)
 #pragma unroll
             for (int e = 0; e < o; ++e) sq[e] += sq[e + o];
         float ss = sq[0];
 #pragma unroll
         for (int o = LPR / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
         const float rinv = 1.0f / sqrtf(ss / (float) D + p.eps);
-        bf16x8 ka, kb, va, vb;
+        out_piece ka, kb, va, vb;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float k0a = bf16r(x[0][e] * rinv * bf(kwa, e));
-            const float k0b = bf16r(x[1][e] * rinv * bf(kwb, e));
+        for (int e = 0; e < E; ++e) {
+            const float k0a = bf16r(x[0][e] * rinv * bf(kwa[e]));
+            const float k0b = bf16r(x[1][e] * rinv * bf(kwb[e]));
             ka[e] = (__bf16) (bf16r(k0a * c[e]) + bf16r(-k0b * s[e]));
             kb[e] = (__bf16) (bf16r(k0b * c[e]) + bf16r(k0a * s[e]));
             va[e] = (__bf16) (x[0][e] * rinv);
             vb[e] = (__bf16) (x[1][e] * rinv);
         }
         if (tt < p.rows) {
-            const size_t at = (size_t) (h0 + g) * p.out_hs + (size_t) t * D + 8 * l;
-            *reinterpret_cast<u32x4_a2 *>(p.k + at) = __builtin_bit_cast(u32x4, ka);
-            *reinterpret_cast<u32x4_a2 *>(p.k + at + HALF) = __builtin_bit_cast(u32x4, kb);
-            *reinterpret_cast<u32x4_a2 *>(p.v + at) = __builtin_bit_cast(u32x4, va);
-            *reinterpret_cast<u32x4_a2 *>(p.v + at + HALF) = __builtin_bit_cast(u32x4, vb);
+            const size_t at = (size_t) (h0 + g) * p.out_hs + (size_t) t * D + E * l;
+            *reinterpret_cast<row_piece *>(p.k + at) = __builtin_bit_cast(row_piece, ka);
+            *reinterpret_cast<row_piece *>(p.k + at + HALF) = __builtin_bit_cast(row_piece, kb);
+            *reinterpret_cast<row_piece *>(p.v + at) = __builtin_bit_cast(row_piece, va);
+            *reinterpret_cast<row_piece *>(p.v + at + HALF) = __builtin_bit_cast(row_piece, vb);
         }
     }
 }
@@ -1063,15 +1064,27 @@ constexpr long long kRawKvWaves = 4 * kTargetGroups;
 
 template <int D, bool Q8>
 void launch_raw_kv(const RawKvParams &p, hipStream_t st) {
-    // Two heads per wave once that leaves a wave for every SIMD, else one: short chunks are
-    // bound by the latency of one wave's work (4 heads x 512 rows 4.2 us with one, 4.7 with
-    // two; x 3000 rows 9.4 with two, 10.3 with four).
-    const long long groups = (p.rows + (1024 / D) - 1) / (1024 / D);  // 64 / (D / 16) rows each
-    const bool wide = groups * ((p.Hkv + 1) / 2) >= kRawKvWaves;
-    const long long waves = groups * (wide ? (p.Hkv + 1) / 2 : p.Hkv);
-    const dim3 grid((unsigned) ((waves + 3) / 4)), block(256);
-    if (wide) hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 2>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 1>), grid, block, 0, st, p);
+    auto waves = [&](int E, int HG) {  // HG heads of 128 E / D rows each
+        const long long groups = (p.rows + (128 * E / D) - 1) / (128 * E / D);
+        return groups * ((p.Hkv + HG - 1) / HG);
+    };
+    auto grid = [&](int E, int HG) { return dim3((unsigned) ((waves(E, HG) + 3) / 4)); };
+    const dim3 block(256);
+    // Fewer waves than SIMDs: a call is one wave's latency, and its E cos / sin most of that (us,
+    // 8 dims a half / fewer): D = 128 one head x 500 rows 3.4 / 2.7 with one row per wave, x 4000
+    // 3.7 / 3.3 (four dims 3.3), x 8000 4.1 / 4.5 (3.8), x 16000 5.0 / 6.8 (5.1); D = 256 x 1000
+    // 3.5 / 2.9, x 4000 4.0 / 3.9 (3.8); D = 512, where a row per wave is four dims, x 500 3.6 /
+    // 3.2, x 4000 5.1 / 5.0, x 8000 7.5 / 8.1.
+    if (waves(8, 1) <= kRawKvWaves / 2)
+        hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 1, D / 128>), grid(D / 128, 1), block, 0, st, p);
+    else if (waves(8, 1) <= kRawKvWaves)
+        hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 1, 4>), grid(4, 1), block, 0, st, p);
+    // Two heads per wave once that leaves a wave for every SIMD (4 heads x 3000 rows 9.4 us with
+    // two, 10.3 with four).
+    else if (waves(8, 2) < kRawKvWaves)
+        hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 1, 8>), grid(8, 1), block, 0, st, p);
+    else
+        hipLaunchKernelGGL((raw_prefill_kv_kernel<D, Q8, 2, 8>), grid(8, 2), block, 0, st, p);
 }
 
 int run_raw_kv(const RawKvParams &p, int D, bool q8, hipStream_t st) {

@@ -381,11 +381,14 @@ def test_raw_q8_prefill_kv_matches_the_oracle():
     _close_bf16(_host(v), ev, "q8 V")
 
 
-@pytest.mark.parametrize("D,Hkv,rows,q8", [(512, 3, 1025, False), (256, 5, 1403, False), (128, 3, 4099, False),
-                                           (512, 3, 1027, True), (512, 1, 1, False)])
+@pytest.mark.parametrize("D,Hkv,rows,q8", [
+    (512, 3, 1025, False), (256, 5, 1403, False), (128, 3, 4099, False), (512, 3, 1027, True),  # two heads a wave
+    (512, 2, 1201, False), (256, 2, 2203, False), (128, 2, 4801, False),                        # one, 8 dims a half
+    (512, 2, 601, True), (256, 2, 1301, False), (128, 3, 2003, False),                          # 4 dims a half
+    (512, 1, 1, False), (512, 2, 33, True), (256, 3, 5, False), (128, 1, 1, False), (128, 2, 37, False),  # a row a wave
+])
 def test_raw_prefill_kv_many_rows(D, Hkv, rows, q8):
-    """Enough rows that a wave takes two kv heads, with an odd head and rows that end inside
-    a wave; inputs and weights at odd element offsets (rows need only element alignment)."""
+    """Each form of the row count's rule, with odd heads and rows that end inside a wave; inputs and weights at odd element offsets (rows need only element alignment)."""
     from apertura_amd.prefill import raw_prefill_kv, raw_q8_prefill_kv
     rng = np.random.default_rng(60 + D + q8)
     raw, kw = _raw_inputs(rng, Hkv, rows, D)
