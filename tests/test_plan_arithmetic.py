@@ -3,7 +3,9 @@ visibility, the prefix table, balanced shares and their segment walk, partial sl
 the merge's split owners, grid splits) -- the functions the attend and merge kernels
 call -- over 3,000 random batches including 256-sequence batches, fewer rows than
 workgroups, and 256 x 16 kv heads x 16,384 workgroups.  tests/plan_check.cpp is built
-with g++; a variant with the batch-256 prefix-table bug planted must fail."""
+with g++; a variant with the batch-256 prefix-table bug planted must fail.  And the plans of
+esda_prefill (apertura_amd/csrc/esda_prefill_plan.h, through tests/prefill_plan_check.cpp):
+the kernel forms and key splits that the GPU tests' shapes rely on."""
 import os
 import shutil
 import subprocess
@@ -15,12 +17,13 @@ SRC = os.path.join(ROOT, "tests", "plan_check.cpp")
 INC = os.path.join(ROOT, "apertura_amd", "csrc")
 
 
-def _build(tmp_path, *defines):
+def _build(tmp_path, *defines, src=SRC):
     cxx = os.environ.get("CXX", "g++")
     if not shutil.which(cxx):
         pytest.skip(f"{cxx} not found")
     exe = tmp_path / ("plan_check" + "".join(d.lower() for d in defines))
-    cmd = [cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-I", INC, SRC, "-o", str(exe)]
+    cmd = [cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-I", INC, "-I", os.path.join(ROOT, "include"),
+           src, "-o", str(exe)]
     cmd += [f"-D{d}" for d in defines]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
@@ -73,3 +76,29 @@ def test_prefill_plan_of_extreme_forced_splits_is_quick():
         _prefill_bytes(16, 8, 256, 64, 2 ** 30, 2 ** 30 - 64, split_keys=32)
     assert _prefill_bytes(16, 8, 256, 2 ** 20, 2 ** 20, 0, split_keys=2 ** 30) == 0
     assert time.perf_counter() - t0 < 2.0
+
+
+def _plans(tmp_path, descs):
+    """The plans of (Hq, Hkv, D, Sq, past, window, split_keys), the chunk's own keys and its past (on
+    sliding layers the last window of it): (waves, rows per tile, splits) each, or the refusal."""
+    exe = _build(tmp_path, src=os.path.join(ROOT, "tests", "prefill_plan_check.cpp"))
+    lines = []
+    for Hq, Hkv, D, Sq, past, window, split in descs:
+        Sk = min(past + Sq, window + Sq) if window else past + Sq
+        lines.append(f"{Hq} {Hkv} {D} {Sq} {Sk} {past} {past + Sq - Sk} {window} {split}")
+    r = subprocess.run([str(exe)], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    out = []
+    for line in r.stdout.splitlines():
+        if line.startswith("refused"):
+            out.append(line)
+        else:
+            nw, qt, tiles, splits, kps, nbytes = map(int, line.split())
+            out.append((nw, qt, splits))
+    return out
+
+
+def test_prefill_forms_the_peak_tests_rely_on(tmp_path):
+    from test_prefill_gpu import PEAKS_512
+    plans = _plans(tmp_path, [(32, 4, 512, Sq, past, 0, 0) for Sq, past, _, _ in PEAKS_512])
+    assert plans == [form for _, _, form, _ in PEAKS_512]

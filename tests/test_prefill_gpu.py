@@ -140,15 +140,25 @@ def test_split_merge_counts(D, Hq, Hkv, Sq, Sk, split_keys):
                 seed=31 + D)
 
 
+# Mid-stream rescales at the two tile heights of head dim 512, 32 query heads over 4: queries, past,
+# the plan's (waves, rows per tile, splits), which tests/test_plan_arithmetic.py holds the plan to,
+# and (head, query, key) peaks.  Every peak lies in a stage after the first of its row's split (four
+# splits of 128 keys; three of 320), so the raised maximum meets sums that are not zero.
+PEAKS_512 = [
+    (64, 448, (4, 64, 4), [(0, 5, 450), (3, 33, 464), (9, 60, 449), (17, 63, 510), (31, 62, 470), (2, 20, 100),
+                           (12, 40, 250), (25, 8, 380)]),
+    (257, 700, (8, 128, 3), [(0, 5, 200), (3, 33, 300), (9, 60, 500), (17, 200, 630), (20, 128, 700), (31, 256, 950),
+                             (6, 100, 64), (14, 255, 400), (27, 16, 713), (1, 256, 940)]),
+]
+
+
 @pytest.mark.parametrize("shared", [True, False])
-@pytest.mark.parametrize("Sq,past", [(64, 448), (600, 424)])
-def test_late_peaks_in_both_tile_heights_at_512(Sq, past, shared):
-    """Mid-stream rescales (as the test above) at the plan's two tile heights of head dim 512: 64
-    queries run four waves on 64-row tiles, 600 eight on 128-row tiles."""
-    Sk = past + Sq
-    peaks = [(h, i, past + i - d) for h, i, d in ((0, 5, 3), (3, 33, 17), (9, 60, 59), (17, Sq - 1, 1), (31, Sq - 2, 40))]
-    rows = sorted({0, 5, 33, 60, 63, Sq - 2, Sq - 1})
-    run_prefill(f"peaks-{Sq}-{int(shared)}", Hq=32, Hkv=4, D=512, Sq=Sq, Sk=Sk, q_pos0=past, k_pos0=0, seed=43,
+@pytest.mark.parametrize("Sq,past,form,peaks", PEAKS_512, ids=["64-rows", "128-rows"])
+def test_late_peaks_in_both_tile_heights_at_512(Sq, past, form, peaks, shared):
+    """The late-peaks test above in the four-wave and the eight-wave kernel (with one K = V buffer
+    the waves of a pair hand each other their rescale factors)."""
+    rows = sorted({0, 63, Sq - 1} | {i for _, i, _ in peaks})
+    run_prefill(f"peaks-{Sq}-{int(shared)}", Hq=32, Hkv=4, D=512, Sq=Sq, Sk=past + Sq, q_pos0=past, k_pos0=0, seed=43,
                 shared=shared, peaks=peaks, rows=rows)
 
 
