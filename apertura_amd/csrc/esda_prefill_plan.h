@@ -53,46 +53,63 @@ ESDA_HD void tile_keys(const PrefillParams &p, int tile, int QT, int &j0, int &j
     j1 = (int) hi;
 }
 
-// A kernel form of one head dim: 16-query blocks per wave, stage halves or not, and its
-// cost in us with one workgroup per CU: `wg` per workgroup (Q and first-stage loads, the
-// pipeline's fill, epilogue) and `stage` per 32-key stage.  Fitted to graph-replayed times
-// over 1 .. 470 stages and 4 .. 512 workgroups; the plans then lie within 5% of the best
-// forced split on 40 of 45 random chunks (the others within 14%).
+// A kernel form of one head dim: 16-query blocks per wave, stage halves or not, waves, and
+// its cost in us: `wg` and `row` per workgroup and query row of it (Q and first-stage loads,
+// the pipeline's fill, epilogue) and `stage` per 32-key stage.  Fitted, with the split's costs
+// below, to graph-replayed times of 12,700 forced (form, split) plans of 1,230 chunks (1 .. 4096
+// queries, past 0 .. 16,000, GQA 1 .. 16, K = V or not); of the forced plans of a chunk the
+// cheapest by this cost then takes 1.008 (D = 128), 1.007 (256) and 1.013 (512) times the
+// fastest's time on average, 1.05, 1.05 and 1.06 at the 95th percentile.
 struct Tiling {
     int qb, kh, nw;
-    float wg, stage;
+    float wg, row, stage;
     int rows() const { return 16 * qb * (kh ? nw / 2 : nw); }
 };
 
-// The forms a head dim can run.  At D = 256, per 32 keys: 64-row stage-halves tiles 0.66 us,
-// 128-row tiles 1.16, and 256-row tiles, whose two blocks share each K and V read, 1.9.  At D =
-// 512 a stage is bound by each wave's own chain, so four waves on 64 rows take nearly as long
-// as eight on 128; but where CUs would idle, the smaller tiles halve what each loads and
-// writes: 32 fresh tokens 15.9 -> 10.1 us, 100 18.6 -> 13.0, 16 over 5016 keys 32.4 -> 28.7, 20 over
-// 973 separate K / V rows 24.5 -> 21.3.
-constexpr Tiling kTilings512[] = {{1, 0, 4, 5.5f, 1.38f}, {1, 0, 8, 9.0f, 1.5f}};
-constexpr Tiling kTilings256[] = {{1, 1, 8, 5.5f, 0.66f}, {1, 0, 8, 5.5f, 1.16f}, {2, 0, 8, 8.0f, 1.9f}};
-constexpr Tiling kTilings128[] = {{2, 0, 8, 3.5f, 1.0f}};
+// The forms a head dim can run, tallest first.  At D = 256, 256-row tiles' two blocks a wave
+// share each K and V read; 64-row tiles split their stages between the wave groups.  At D = 512
+// a stage is bound by each wave's own chain, so four waves on 64 rows take nearly as long as
+// eight on 128; but where CUs would idle, the smaller tiles halve what each loads and writes:
+// 32 fresh tokens 15.9 -> 10.1 us, 100 18.6 -> 13.0, 16 over 5016 keys 32.4 -> 28.7, 20 over 973
+// separate K / V rows 24.5 -> 21.3.
+constexpr Tiling kTilings512[] = {{1, 0, 8, 5.6f, 0.074f, 1.52f}, {1, 0, 4, 6.2f, 0.070f, 1.39f}};
+constexpr Tiling kTilings256[] = {{2, 0, 8, 7.0f, 0.037f, 1.457f}, {1, 0, 8, 5.0f, 0.037f, 0.95f},
+                                  {1, 1, 8, 6.0f, 0.049f, 0.6f}};
+constexpr Tiling kTilings128[] = {{2, 0, 8, 5.1f, 0.018f, 1.01f}};
 
-// Estimated us of a plan: `pieces(f)` calls f(stages) for each workgroup of one kv head in
-// dispatch order.  The heads run side by side, so one head has kTargetGroups / Hkv CUs; the
-// dispatcher hands a workgroup to the CU that falls idle first, which for the descending
-// lengths of the tiles (latest first) is the order back and forth over the CUs.
-template <class F>
-float makespan(int Hkv, const Tiling &t, F &&pieces) {
-    const int cus = std::max(1, kTargetGroups / Hkv);
-    const float share = Hkv > kTargetGroups ? (float) Hkv / kTargetGroups : 1.0f;  // heads per CU
-    float load[kTargetGroups];
-    std::fill_n(load, cus, 0.0f);
-    int at = 0, dir = 1;
-    pieces([&](int stages) {
-        load[at] += t.wg + stages * t.stage;
-        if (at + dir < 0 || at + dir >= cus) dir = -dir;  // the end takes two in a row
-        else at += dir;
-    });
+constexpr int kXcds = 8, kEngines = 4, kEngineCus = kTargetGroups / (kXcds * kEngines);
+constexpr float kEmptyUs = 1.2f;  // a workgroup whose split holds no key of its tile
+
+// Estimated us until the last workgroup of a plan ends.  Whatever their lengths, workgroup i
+// goes to XCD i % 8 and an XCD's workgroups in turn to its four engines of 8 CUs, each to the CU
+// that falls idle first, none before the one ahead of it on the XCD.  With 2 (kv head, split)
+// pairs a tile per XCD, or 1 of 4 or 8 in all, some engines or XCDs then get all the long
+// workgroups: 2705 queries over 3739 keys at D = 128, 85 tiles of one head, take 89 us in 4
+// splits and 62 in 3; 2043 fresh ones, 32 tiles of 8 heads, 77 unsplit and 100 in 2.  (Any CU
+// of the GPU, or of the XCD, to the next workgroup: 52 and 73 us estimated for those two.)
+// nst: stages of each tile, latest first; last_rows: query rows of the latest tile.
+inline float makespan(const Tiling &t, const int *nst, int tiles, int last_rows, int Hkv, int splits, int per) {
+    float ends[kXcds][kEngines][kEngineCus] = {}, front[kXcds] = {};
     float most = 0.0f;
-    for (int i = 0; i < cus; ++i) most = std::max(most, load[i]);
-    return most * share;
+    unsigned wg = 0;
+    for (int i = 0; i < tiles; ++i)
+        for (int s = 0; s < splits; ++s) {
+            const int n = std::min(per, nst[i] - s * per);
+            const float us = n > 0 ? t.wg + t.row * (i ? t.rows() : last_rows) + n * t.stage : kEmptyUs;
+            for (int h = 0; h < Hkv; ++h, ++wg) {
+                const unsigned xcd = wg % kXcds;
+                float *e = ends[xcd][wg / kXcds % kEngines];
+                unsigned cu = wg / (kXcds * kEngines);
+                if (cu >= kEngineCus) {
+                    cu = 0;
+                    for (int c = 1; c < kEngineCus; ++c) cu = e[c] < e[cu] ? c : cu;
+                    front[xcd] = std::max(front[xcd], e[cu]);
+                }
+                e[cu] = front[xcd] + us;
+                most = std::max(most, e[cu]);
+            }
+        }
+    return most;
 }
 
 // Splitting adds a dependent launch and D fp32 per row and split, written by the attention
@@ -102,7 +119,9 @@ float makespan(int Hkv, const Tiling &t, F &&pieces) {
 // L2s together (8 x 4 MB) the write-back overlaps the kernel, and waiting for memory costs
 // more: 32 MB 46.7 -> 45.7 us, 40 MB 43.7 both ways, 48 MB 42.2 -> 46.4, 64 MB 42.2 -> 54.0.
 constexpr float kPartNtBytes = 36.0e6f;
-inline float split_cost(float part_bytes) { return 5.0f + 3.1e-7f * part_bytes; }  // us
+inline float split_cost(float part_bytes, int splits) {  // us
+    return 3.0f + 2.2e-7f * part_bytes + 0.15f * std::max(0, splits - 8);
+}
 constexpr int kMaxRounds = 3;  // split plans of more workgroups per CU only add partials
 
 // Validates a description and fills the kernel parameters' shape fields and plan.  Returns
@@ -146,9 +165,8 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
     p->o_hs = d->out_head_stride;
     p->scale_log2e = d->scale * 1.4426950408889634f;
     // Form and split: the cheapest by the cost above.  What counts is how the workgroups fill
-    // rounds of 256 CUs: 333 queries over 5933 keys (84 tiles) take 135 us as 252 workgroups
-    // and 192 us as 336, whose second round is mostly idle; 770 fresh tokens (192 tiles) 51 us
-    // unsplit and 80 us split in two.
+    // rounds of 256 CUs: 333 queries over 5933 keys (K = V, 84 tiles) take 126 us as 252
+    // workgroups and 190 as 336, whose second round is mostly idle.
     const long long rows = (long long) d->seq_q * p->G;
     const Tiling *forms = D == 512 ? kTilings512 : D == 256 ? kTilings256 : kTilings128;
     const int nforms = D == 512 ? 2 : D == 256 ? 3 : 1;
@@ -159,12 +177,13 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         const int QT = t.rows();
         const long long tiles = (rows + QT - 1) / QT, groups = tiles * d->num_kv_heads;
         if (groups > (1LL << 24)) {
-            if (f + 1 < nforms) continue;
+            if (f) break;
             return "esda_prefill: too many query tiles";
         }
         const bool few = groups <= kMaxRounds * kTargetGroups;
         int nst[kMaxRounds * kTargetGroups];  // few: stages of each tile, latest first
-        int most = 1;
+        const int last_rows = (int) (rows - (tiles - 1) * QT);
+        int most = 1, most_full = 0;  // stages of the longest tile, and of those of QT rows
         double total = 0.0;
         for (int i = 0; i < (int) tiles; ++i) {
             int a, b;
@@ -172,22 +191,33 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
             const int n = (int) (((long long) b - a + kStageKeys - 1) / kStageKeys);
             if (few) nst[i] = n;
             most = std::max(most, n);
-            total += t.wg + n * t.stage;
+            if (i || last_rows == QT) most_full = std::max(most_full, n);
+            total += t.wg + t.row * (i ? QT : last_rows) + n * t.stage;
         }
+        const float even = (float) (total * d->num_kv_heads / kTargetGroups);
         auto consider = [&](int per) {  // per: stages per split
             const int splits = (most + per - 1) / per;
-            float us = splits > 1 ? split_cost(4.0f * D * (float) rows * d->num_kv_heads * splits) : 0.0f;
+            float us = splits > 1 ? split_cost(4.0f * D * (float) rows * d->num_kv_heads * splits, splits) : 0.0f;
+            const float longest = std::max(t.wg + t.row * last_rows + std::min(per, most) * t.stage,
+                                           most_full ? t.wg + t.row * QT + std::min(per, most_full) * t.stage : 0.0f);
             // no plan is faster than its longest workgroup, nor than its work spread evenly
-            if (us + std::max(t.wg + std::min(per, most) * t.stage,
-                              (float) (total * d->num_kv_heads / kTargetGroups)) >= best)
-                return splits;
-            if (few && tiles * splits <= 2LL * kMaxRounds * kTargetGroups)
-                us += makespan(d->num_kv_heads, t, [&](auto &&piece) {
-                    for (int i = 0; i < (int) tiles; ++i)
-                        for (int j = 0; j < nst[i]; j += per) piece(std::min(per, nst[i] - j));
-                });
-            else  // many workgroups: the CUs stay busy but for the end of the last round
-                us += (float) (total * d->num_kv_heads / kTargetGroups) + 0.5f * (t.wg + most * t.stage);
+            if (us + std::max(longest, even) >= best) return;
+            if (groups * splits <= kTargetGroups) {
+                us += longest;  // one round
+            } else if (few && groups * splits <= 2LL * kMaxRounds * kTargetGroups) {
+                // nor than its pieces' work spread evenly, nor the rounds that its whole pieces take
+                int whole = 0, pieces = 0;
+                for (int i = 0; i < (int) tiles; ++i) {
+                    whole += nst[i] / per;
+                    pieces += (nst[i] + per - 1) / per;
+                }
+                const int rounds = (whole * d->num_kv_heads + kTargetGroups - 1) / kTargetGroups;
+                const float spread = even + (float) (pieces - tiles) * d->num_kv_heads * t.wg / kTargetGroups;
+                if (us + std::max(spread, rounds * (t.wg + per * t.stage)) >= best) return;
+                us += makespan(t, nst, (int) tiles, last_rows, d->num_kv_heads, splits, per);
+            } else {  // many workgroups: the CUs stay busy but for the end of the last round
+                us += even + 0.5f * (t.wg + t.row * QT + most * t.stage);
+            }
             if (us < best) {
                 best = us;
                 kps = per * kStageKeys;
@@ -197,15 +227,19 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
                 p->nw = t.nw;
                 p->tiles = (int) tiles;
             }
-            return splits;
         };
         if (d->split_keys > 0) {
             consider(d->split_keys / kStageKeys);
         } else {
             consider(most);
-            for (int s = 2; s <= most && groups * s <= kMaxRounds * kTargetGroups;)
-                s = std::max(s, consider((most + s - 1) / s)) + std::max(1, s / 4);
+            int last = most;
+            for (int s = 2; s <= most && groups * s <= kMaxRounds * kTargetGroups; s += std::max(1, s / 4)) {
+                const int per = (most + s - 1) / s;
+                if (per != last) consider(per);
+                last = per;
+            }
         }
+        if (!few) break;  // many rounds of the tallest tiles: nothing for shorter ones to fill
     }
     if (d->split_keys > 0) kps = d->split_keys;
     const long long splits = ((long long) most_stages * kStageKeys + kps - 1) / kps;

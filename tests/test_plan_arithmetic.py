@@ -50,10 +50,10 @@ def _prefill_bytes(Hq, Hkv, D, Sq, Sk, q_pos0, k_pos0=0, window=0, split_keys=0)
 
 
 @pytest.mark.parametrize("Hq,Hkv,D,Sq,past,splits", [
-    (32, 4, 512, 333, 5600, 3),    # 84 tiles: 252 workgroups, not 336
-    (32, 4, 512, 200, 8056, 4),    # 52 tiles: 208
+    (32, 4, 512, 333, 5600, 3),    # 84 tiles of 4 heads: 252 workgroups, not 336
+    (32, 4, 512, 200, 8056, 4),    # 52 tiles of 4 heads: 208
     (32, 4, 512, 512, 15872, 2),   # 128 tiles: 256
-    (32, 4, 512, 770, 0, 1),       # 196 fresh tiles: unsplit
+    (32, 4, 512, 770, 0, 1),       # 388 fresh workgroups of four waves: unsplit
     (32, 4, 512, 4096, 0, 1),      # four rounds of tiles
     (8, 4, 256, 17, 10, 1),        # one stage
 ])
@@ -102,3 +102,13 @@ def test_prefill_forms_the_peak_tests_rely_on(tmp_path):
     from test_prefill_gpu import PEAKS_512
     plans = _plans(tmp_path, [(32, 4, 512, Sq, past, 0, 0) for Sq, past, _, _ in PEAKS_512])
     assert plans == [form for _, _, form, _ in PEAKS_512]
+
+
+def test_prefill_forms_the_planned_tests_rely_on(tmp_path):
+    """Forms and splits at the edges of the choice; among them chunks that the dispatch order
+    decides (round-robin over the XCDs and their engines, whatever the workgroups' lengths)."""
+    from test_prefill_gpu import PLANNED
+    plans = _plans(tmp_path, [(Hq, Hkv, D, Sq, past, window, 0) for D, Hq, Hkv, Sq, past, window, _ in PLANNED])
+    assert plans == [form for *_, form in PLANNED]
+    # unsplit, though an even spread of two splits' work would end first
+    assert _plans(tmp_path, [(32, 8, 128, 2043, 0, 0, 0), (16, 16, 512, 1364, 91, 0, 0)]) == [(8, 256, 1), (4, 64, 1)]

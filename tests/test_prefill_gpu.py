@@ -162,18 +162,26 @@ def test_late_peaks_in_both_tile_heights_at_512(Sq, past, form, peaks, shared):
                 shared=shared, peaks=peaks, rows=rows)
 
 
-@pytest.mark.parametrize("D,Hq,Hkv,Sq,past,window", [
-    (512, 32, 4, 257, 700, 0),     # 17 tiles a head, the last of 8 rows: three splits fill one round
-    (512, 16, 2, 16, 4900, 0),     # one full tile a head: tens of splits
-    (512, 8, 8, 129, 0, 0),        # fresh, a last tile of one row
-    (512, 2, 1, 33, 3000, 0),      # two 64-row tiles, the last of two rows, many splits
-    (256, 32, 16, 1100, 0, 256),   # 128-row tiles just past one round of the CUs
-    (256, 16, 8, 17, 2000, 1024),  # short chunk: stage halves and splits together
-    (256, 16, 8, 2470, 0, 1024),   # 128-row tiles in two uneven rounds
-    (256, 32, 16, 4001, 1341, 1024),  # 256-row tiles, stages off the grid, a short last tile
-    (128, 8, 4, 300, 1500, 0),     # 256-row tiles with splits
-])
-def test_planned_forms_and_splits(D, Hq, Hkv, Sq, past, window):
+# Shapes at the edges of the form and split choice with the plan's (waves, rows per tile, splits),
+# which tests/test_plan_arithmetic.py holds it to: every form of a head dim, unsplit and split.
+PLANNED = [
+    (512, 32, 4, 257, 700, 0, (8, 128, 3)),      # 17 tiles a head, the last of 8 rows: three splits fill one round
+    (512, 16, 2, 16, 4900, 0, (4, 64, 31)),      # two 64-row tiles a head, many splits
+    (512, 8, 8, 129, 0, 0, (4, 64, 1)),          # fresh, a last tile of one row
+    (512, 2, 1, 33, 3000, 0, (4, 64, 24)),       # two 64-row tiles, the last of two rows
+    (512, 32, 4, 600, 424, 0, (8, 128, 1)),      # 152 workgroups of eight waves, not 300 of four
+    (256, 32, 16, 1100, 0, 256, (8, 128, 1)),    # 128-row tiles just past one round of the CUs
+    (256, 16, 8, 17, 2000, 1024, (8, 128, 11)),  # one tile a head, splits
+    (256, 16, 8, 70, 700, 1024, (8, 64, 7)),     # stage halves and splits, a last tile of 12 rows
+    (256, 16, 8, 2470, 0, 1024, (8, 128, 1)),    # 128-row tiles in two uneven rounds
+    (256, 32, 16, 4001, 1341, 1024, (8, 256, 1)),  # stages off the grid, a short last tile
+    (128, 8, 4, 300, 1500, 0, (8, 256, 12)),
+    (128, 8, 1, 2705, 1034, 0, (8, 256, 3)),     # 85 tiles of one head: with four splits two XCDs get all whole ones
+]
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,Sq,past,window,form", PLANNED)
+def test_planned_forms_and_splits(D, Hq, Hkv, Sq, past, window, form):
     """Automatic plans at the edges of the form and split choice: sampled rows (the first and
     last of the chunk, of its tiles and of the tiles' ragged end)."""
     Sk = min(past + Sq, window + Sq) if window else past + Sq
