@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
     const int lane = threadIdx.x & 63;
     const long long nrows = (long long) p.Sq * p.Hq;
-    const long long wv = (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+    const long long wv = p.merge_wave0 + (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
     if (wv >= nrows * PARTS) return;
     const long long row = wv / PARTS;
     const int d0 = (int) (wv % PARTS) * 64 * VEC + lane * VEC;
@@ -848,11 +848,15 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
             hipLaunchKernelGGL((prefill_kernel<256, 1>), grid, block, 0, st, p);
     }
     if ((stages & 2) && p.splits > 1) {
-        const long long waves = (long long) p.Sq * p.Hq * (D >= 256 ? D / 256 : 1);
-        const dim3 grid((unsigned) ((waves + 3) / 4)), block(256);
-        if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, p);
-        else if (p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((prefill_merge_kernel<D, 0>), grid, block, 0, st, p);
+        const long long waves = merge_waves(p, D);
+        PrefillParams mp = p;
+        for (mp.merge_wave0 = 0; mp.merge_wave0 < waves; mp.merge_wave0 += kMergeLaunchWaves) {
+            const long long n = std::min(kMergeLaunchWaves, waves - mp.merge_wave0);
+            const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
+            if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, mp);
+            else if (p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8>), grid, block, 0, st, mp);
+            else hipLaunchKernelGGL((prefill_merge_kernel<D, 0>), grid, block, 0, st, mp);
+        }
     }
 }
 

@@ -31,6 +31,7 @@ struct PrefillParams {
     int kh;                  // 1: the two wave groups split each tile's stages (even / odd)
     int nw;                  // waves per workgroup (query tile: 16 qb nw rows, half of it with kh)
     int part_nt;             // 1: partials stored non-temporal
+    long long merge_wave0;   // the split merge's launch: its first wave
 };
 
 // Query row r of a GQA group's rows -> its position in the chunk (r % G is its head).  At
@@ -250,6 +251,11 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
     p->part_nt = 4.0f * D * p->Sq * p->Hq * p->splits <= kPartNtBytes;
     return nullptr;
 }
+
+// Waves of the split merge: one per query row of up to 256 dims, and as many as a launch takes
+// (2^31 threads; a HIP launch holds fewer than 2^32).  More rows take several launches.
+constexpr long long kMergeLaunchWaves = 1LL << 25;
+inline long long merge_waves(const PrefillParams &p, int D) { return (long long) p.Sq * p.Hq * (D == 512 ? 2 : 1); }
 
 inline size_t workspace_of(const PrefillParams &p, int D) {
     if (p.splits <= 1) return 0;

@@ -140,6 +140,29 @@ def test_split_merge_counts(D, Hq, Hkv, Sq, Sk, split_keys):
                 seed=31 + D)
 
 
+def test_split_merge_of_more_rows_than_a_launch_holds():
+    """2^26 + 2^20 query rows at head dim 128 in three splits: the merge's wave per row is more threads
+    than one launch takes.  Every head has the same query (head stride 0), so each position's
+    output is checked once against the oracle and every head against the first."""
+    from apertura_amd.prefill import PrefillStep, prefill, prefill_workspace_bytes
+    Hq, Sq, D = 2 ** 20, 65, 128
+    rng = np.random.default_rng(91)
+    q, k, v = rms_rows(rng, (1, Sq, D)), rms_rows(rng, (1, Sq, D)), rms_rows(rng, (1, Sq, D))
+    step = PrefillStep(Hq, 1, D, Sq, Sq, 0, 0, scale=D ** -0.5, split_keys=32, q_head_stride=0, q_row_stride=D)
+    need = prefill_workspace_bytes(step) + 2 * Sq * Hq * D
+    if torch.cuda.mem_get_info()[0] < need + 2 ** 33:
+        pytest.skip(f"needs {need >> 30} GiB of device memory")
+    out = prefill(step, _dev(q), _dev(k), _dev(v))
+    torch.cuda.synchronize()
+    ref = orc.prefill_f64(q, k, v, 0, 0, 0, D ** -0.5)  # [Sq, 1, D]
+    err = np.abs(orc.from_bf16(_host(out[:, :1])).astype(np.float64) - ref)
+    assert err.max() <= TOL_MAX and err.mean() <= TOL_MEAN
+    for i in range(Sq):
+        assert bool((out[i] == out[i, :1]).all()), f"position {i}"
+    del out
+    torch.cuda.empty_cache()
+
+
 # Mid-stream rescales at the two tile heights of head dim 512, 32 query heads over 4: queries, past,
 # the plan's (waves, rows per tile, splits), which tests/test_plan_arithmetic.py holds the plan to,
 # and (head, query, key) peaks.  Every peak lies in a stage after the first of its row's split (four
