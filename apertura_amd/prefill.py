@@ -91,11 +91,13 @@ def prefill(step: PrefillStep, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     if out is None:
         out = torch.empty((step.seq_q, step.num_q_heads, D), dtype=bf, device=q.device)
     d = step.desc()
-    # the extent each tensor must cover (elements), checked before the pointers go down
-    kv = (d.num_kv_heads - 1) * d.kv_head_stride + d.seq_k * D
-    for name, t, need in (("q", q, (d.num_q_heads - 1) * d.q_head_stride + (d.seq_q - 1) * d.q_row_stride + D),
-                          ("k", k, kv), ("v", v, kv),
-                          ("out", out, (d.seq_q - 1) * d.out_row_stride + (d.num_q_heads - 1) * d.out_head_stride + D)):
+    # the extent each tensor must cover (elements), checked before the pointers go down; by the
+    # step's own sizes, which the description's 32-bit fields would wrap
+    kv = (step.num_kv_heads - 1) * d.kv_head_stride + step.seq_k * D
+    for name, t, need in (
+            ("q", q, (step.num_q_heads - 1) * d.q_head_stride + (step.seq_q - 1) * d.q_row_stride + D),
+            ("k", k, kv), ("v", v, kv),
+            ("out", out, (step.seq_q - 1) * d.out_row_stride + (step.num_q_heads - 1) * d.out_head_stride + D)):
         if t.dtype != bf or not t.is_cuda:
             raise ValueError(f"{name} must be a bf16 GPU tensor")
         if t.untyped_storage().nbytes() // 2 - t.storage_offset() < need:
