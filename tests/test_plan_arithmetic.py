@@ -112,3 +112,37 @@ def test_prefill_forms_the_planned_tests_rely_on(tmp_path):
     assert plans == [form for *_, form in PLANNED]
     # unsplit, though an even spread of two splits' work would end first
     assert _plans(tmp_path, [(32, 8, 128, 2043, 0, 0, 0), (16, 16, 512, 1364, 91, 0, 0)]) == [(8, 256, 1), (4, 64, 1)]
+
+
+def test_plans_follow_the_description_of_each_call(tmp_path):
+    """The library keeps the calling thread's last plan: descriptions that differ in one field, taken
+    in turn and from two threads at once, get their own workspace sizes, refused ones none."""
+    import threading
+
+    from apertura_amd import EsdaError
+    base = dict(Hq=32, Hkv=4, D=512, Sq=200, Sk=8256, q_pos0=8056)
+    descs = [base, dict(base, Sq=199, q_pos0=8057), dict(base, split_keys=512), dict(base, window=1024),
+             dict(base, D=256)]
+    exe = _build(tmp_path, src=os.path.join(ROOT, "tests", "prefill_plan_check.cpp"))
+    text = "".join(f"{d['Hq']} {d['Hkv']} {d['D']} {d['Sq']} {d['Sk']} {d['q_pos0']} 0 {d.get('window', 0)} "
+                   f"{d.get('split_keys', 0)}\n" for d in descs)
+    r = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60)
+    want = [int(line.split()[-1]) for line in r.stdout.splitlines()]
+    assert len(set(want)) == len(want)
+    wrong = []
+
+    def walk(order):
+        for i in order:
+            if _prefill_bytes(**descs[i]) != want[i] or _prefill_bytes(**descs[i]) != want[i]:
+                wrong.append(i)
+            with pytest.raises(EsdaError):
+                _prefill_bytes(**dict(descs[i], split_keys=33))
+            if _prefill_bytes(**descs[i]) != want[i]:
+                wrong.append(i)
+
+    threads = [threading.Thread(target=walk, args=(list(range(len(descs)))[::s] * 50,)) for s in (1, -1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
