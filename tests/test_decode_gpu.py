@@ -293,13 +293,18 @@ EDGE = [
     # plan C5's global layers use): here far fewer visible rows than shares, with one
     # empty-ish sequence
     dict(name="balanced_256_shares_tiny", B=3, Hq=16, Hkv=2, D=512, cap=8192, shared=True, pos=[0, 40, 300]),
-    # merge_kernel over balanced shares: 4 pairs of about 64 partials (one of over 128: its loop),
-    # 40 pairs of about 6, and 44 (the last of its range: 42 pairs), where merge_rows_kernel takes over
+    # merge_kernel over balanced shares (tests/test_plan_arithmetic.py holds each case's merge and
+    # its longest pair to what is said here): 4 pairs of up to 117 partials, 40 pairs of 12.8 on
+    # average, 42 of 6.1 (the last of its range), and 44, where merge_rows_kernel takes over
     dict(name="balanced_merge_4_pairs", B=2, Hq=16, Hkv=2, D=512, cap=20000, shared=True, pos=[19999, 2000]),
     dict(name="balanced_merge_40_pairs", B=10, Hq=8, Hkv=4, D=256, cap=3000,
          pos=[2999, 0, 17, 900, 1500, 2200, 64, 2998, 1, 333]),
     dict(name="balanced_merge_42_pairs", B=14, Hq=6, Hkv=3, D=128, cap=1200, pos=[80 * i + 5 for i in range(14)]),
     dict(name="balanced_merge_44_pairs", B=11, Hq=8, Hkv=4, D=128, cap=1500, pos=[130 * i + 3 for i in range(11)]),
+    # pairs of more partials than the merge's threads hold in registers, which loop over them: 252 of
+    # 64 (merge_kernel<4>, picked by the average share), and 511 of 256 (merge_kernel<16>)
+    dict(name="balanced_merge_loop_4", B=8, Hq=8, Hkv=1, D=512, cap=20000, shared=True, pos=[19999] + [50] * 7),
+    dict(name="balanced_merge_loop_16", B=2, Hq=4, Hkv=1, D=256, cap=20000, pos=[19999, 50]),
 ]
 
 

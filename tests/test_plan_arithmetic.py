@@ -146,3 +146,37 @@ def test_plans_follow_the_description_of_each_call(tmp_path):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("name,merge,longest", [
+    ("balanced_merge_4_pairs", "merge_kernel<16>", 117),
+    ("balanced_merge_40_pairs", "merge_kernel<4>", 36),
+    ("balanced_merge_42_pairs", "merge_kernel<4>", 13),
+    ("balanced_merge_44_pairs", "merge_rows_kernel", 13),
+    ("balanced_merge_loop_4", "merge_kernel<4>", 252),
+    ("balanced_merge_loop_16", "merge_kernel<16>", 511),
+])
+def test_balanced_merges_the_edge_cases_rely_on(name, merge, longest):
+    """The merge and the most partials of a pair for the GPU tests' balanced cases: the plan's shares
+    from the workspace it asks for, the owners by esda_plan.h's rule, the merge by the launch's."""
+    from apertura_amd.decode import DecodeStep, workspace_bytes
+    from test_decode_gpu import EDGE
+    c = next(c for c in EDGE if c["name"] == name)
+    B, Hkv, D, cap = c["B"], c["Hkv"], c["D"], c["cap"]
+    G = c["Hq"] // Hkv
+    n = workspace_bytes(DecodeStep(batch=B, num_q_heads=c["Hq"], num_kv_heads=Hkv, head_dim=D, cap=cap,
+                                   kv_shared=c.get("shared", False), scale=1.0))
+    up = lambda x: (x + 255) // 256 * 256
+    W = next(w for w in range(1, 20000) if 256 + up((B + 1) * 8) + up((B * Hkv + w) * G * 8) + (B * Hkv + w) * G * D * 4 == n)
+    pairs, rows = B * Hkv, [p + 1 for p in c["pos"]]
+    total = sum(rows) * Hkv
+    Wr, first, most = min(W, total), 0, 0
+    for r in rows:
+        for _ in range(Hkv):
+            owner = lambda x: ((x + 1) * Wr - 1) // total
+            most = max(most, owner(first + r - 1) - owner(first) + 1)
+            first += r
+    kernel = "merge_rows_kernel" if W < 6 * pairs else "merge_kernel<4>" if 2 * W <= 64 * pairs else "merge_kernel<16>"
+    assert (kernel, most) == (merge, longest)
+    if "loop" in name:
+        assert most > (64 if kernel == "merge_kernel<4>" else 256)
