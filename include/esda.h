@@ -165,7 +165,8 @@ typedef struct esda_raw_args {
     size_t workspace_bytes;
     const void *rope_table;  /* optional, NULL: computed in the kernel.  [rope_table_rows][64]
                                 u32 from esda_rope_table (cos / sin of row*inv_freq[d]):
-                                the same values and outputs, read instead of computed   */
+                                the values the kernel otherwise computes (outputs agree
+                                to fp32 rounding: other summation orders)              */
     int32_t rope_table_rows; /* >= cap when rope_table is set                          */
 } esda_raw_args;
 

@@ -104,8 +104,8 @@ def run_raw(name, *, B=1, Hq=32, Hkv=4, cap, pos, scale=1.0, seed=0, split_rows=
     return o, errs
 
 
-# table=True is the ES layer's form (precomputed rotary table): the wave-private-ring kernel;
-# table=False the 8-wave kernel that computes its cos / sin.
+# table=True is the ES layer's form (precomputed rotary table); table=False the form of the same
+# kernel that computes its cos / sin.
 TABLE = pytest.mark.parametrize("table", [False, True], ids=["own-sincos", "table"])
 
 
@@ -130,10 +130,10 @@ def test_raw_long_context_131072_with_rope_table():
 
 
 def test_rope_table_kernels_agree_and_the_table_matches_fp64():
-    """Decode with the precomputed table (the wave-private-ring kernel) and with the kernel's
-    own cos/sin (the 8-wave kernel) over ragged batched positions with an append: each
-    within the tolerance of the fp64 oracle and of each other (their fp32 sums run in
-    different orders, so they are not bit-identical); the table entries equal bf16(cos /
+    """Decode with the precomputed table and with the kernel's own cos/sin over ragged batched
+    positions with an append: each within the tolerance of the fp64 oracle and of each other
+    (the two forms add a row's squares, and their shares' partials, in different orders, so they
+    are not bit-identical); the table entries equal bf16(cos /
     sin) of the fp32 angle but for rare rounding-boundary cases."""
     from apertura_amd.decode import RawStep, decode_raw, new_raw_workspace, rope_table
     rng = np.random.default_rng(23)
@@ -362,3 +362,23 @@ def test_raw_own_sincos_shares_of_short_sequences(B, Hkv, pos):
     """Without a table the shares of a balanced plan count a start-up cost per pair beside its
     rows: segments, partials and the merge's owners of sequences far shorter than that cost."""
     run_raw(f"short-{B}", B=B, Hq=8 * Hkv, Hkv=Hkv, cap=200, pos=pos, scale=512 ** -0.5, seed=80 + B)
+
+
+@pytest.mark.parametrize("cap,pos,split_rows", [(4096, 4095, 0), (1024, 1000, 16), (512, 37, 0), (20000, 17777, 0)])
+def test_raw_table_and_own_sincos_outputs(cap, pos, split_rows):
+    """One sequence with the table and without: the same cos / sin values and splits, so the outputs
+    differ by the row norms' last bits alone.  Two ulps of a norm flip the bf16 rounding of 1 K
+    element in 2^14 by 2^-8, a score by some 1e-5, and so the rounding of 0.5% of the outputs:
+    2e-4 relative (2.4e-4 to 3.1e-4 seen); the bar is 1e-3.  A cos / sin row or frequency of another position moves one
+    weight of n by about its own size, 1 / sqrt(n) relative (5e-3 or more here)."""
+    from apertura_amd.decode import RawStep, decode_raw, new_raw_workspace, rope_table
+    rng = np.random.default_rng(95 + cap)
+    q, raw, kn, kw = _raw_inputs(rng, 1, 32, 4, cap)
+    inv_d = torch.from_numpy(orc.rope_inv_freq(512, 1e6, 0.25)).cuda()
+    step = RawStep(batch=1, num_q_heads=32, num_kv_heads=4, cap=cap, eps=EPS, scale=512 ** -0.5, split_rows=split_rows)
+    p = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    a, b = (decode_raw(step, _dev(q), _dev(kn), _dev(raw), p, _dev(kw), inv_d, workspace=new_raw_workspace(step, "cuda"),
+                       rope_table=t).float() for t in (None, rope_table(inv_d, cap)))
+    rel = float((a - b).norm() / b.norm())
+    print(f"[raw] table against own cos / sin, {pos + 1} rows: rel {rel:.2e}, {float((a != b).float().mean()):.2%} differ", flush=True)
+    assert rel <= 1e-3

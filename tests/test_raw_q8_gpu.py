@@ -102,8 +102,8 @@ def run_q8(name, *, B=1, Hq=32, Hkv=4, cap, pos, scale=1.0, seed=0, split_rows=0
     return o, errs
 
 
-# table=True is the ES layer's form (precomputed rotary table): the wave-private-ring kernel;
-# table=False the 8-wave kernel that computes its cos / sin.
+# table=True is the ES layer's form (precomputed rotary table); table=False the form of the same
+# kernel that computes its cos / sin.
 TABLE = pytest.mark.parametrize("table", [False, True], ids=["own-sincos", "table"])
 
 
@@ -118,7 +118,7 @@ def test_q8_in_model_scale_one(table):
 
 
 def test_q8_long_context_131072():
-    """The C4 shape over a q8 raw stream: 131072 rows (the 8-wave kernel, its own cos / sin)."""
+    """The C4 shape over a q8 raw stream: 131072 rows, the kernel computing its cos / sin."""
     run_q8("c4-q8", cap=131072, pos=[131071], scale=512 ** -0.5, seed=5)
 
 
@@ -187,10 +187,10 @@ def test_q8_long_context_131072_with_rope_table():
 
 
 def test_q8_table_and_own_sincos_kernels_agree():
-    """q8 decode with the precomputed table (the wave-private-ring kernel) and with the
-    kernel's own cos/sin (the 8-wave kernel), over ragged batched positions with the new rows
-    quantized in: the quantized cache bytes are identical, and each output is within the
-    tolerance of the fp64 q8 oracle and of the other (different fp32 summation orders)."""
+    """q8 decode with the precomputed table and with the kernel's own cos/sin, over ragged batched
+    positions with the new rows quantized in: the quantized cache bytes are identical, and each
+    output is within the tolerance of the fp64 q8 oracle and of the other (other shares, and
+    quotients where the table form takes reciprocals)."""
     from apertura_amd.decode import decode_raw_q8, new_raw_workspace, q8_step_for, rope_table
     rng = np.random.default_rng(33)
     B, cap = 2, 4096
@@ -264,3 +264,28 @@ def test_q8_own_sincos_shares_of_short_sequences(B, Hkv, pos):
     """Without a table the shares of a balanced plan count a start-up cost per pair beside its
     rows: segments, partials and the merge's owners of sequences far shorter than that cost."""
     run_q8(f"short-{B}", B=B, Hq=8 * Hkv, Hkv=Hkv, cap=200, pos=pos, scale=512 ** -0.5, seed=80 + B)
+
+
+@pytest.mark.parametrize("cap,pos,split_rows", [(4096, 4095, 0), (1024, 1000, 16), (512, 37, 0), (20000, 17777, 0)])
+def test_q8_table_and_own_sincos_outputs(cap, pos, split_rows):
+    """One q8 sequence with the table and without: the same cos / sin values, K and splits; the weight
+    factors differ by an ulp (divisions against reciprocals), which moves the bf16 rounding of few
+    outputs.  The bar and what it catches are those of the raw form's test."""
+    from apertura_amd.decode import decode_raw_q8, new_raw_workspace, q8_step_for, rope_table
+    rng = np.random.default_rng(97 + cap)
+    qc, sc, bs = orc.quantize_rows(_raw_rows(rng, (1, 4, cap, 512)))
+    q = orc.rms_norm_rows(orc.to_bf16(rng.standard_normal((1, 32, 512), dtype=np.float32)), None, 1e-6)
+    kn = _raw_rows(rng, (1, 4, 512))
+    kw = orc.to_bf16((1.0 + 0.25 * rng.standard_normal(512)).astype(np.float32))
+    inv_d = torch.from_numpy(orc.rope_inv_freq(512, 1.0e6, 0.25)).cuda()
+    p = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    outs = []
+    for t in (None, rope_table(inv_d, cap)):
+        q8_d = torch.from_numpy(qc).cuda()
+        step = q8_step_for(q8_d, 32, eps=EPS, scale=512 ** -0.5, split_rows=split_rows)
+        outs.append(decode_raw_q8(step, _dev(q), _dev(kn), q8_d, torch.from_numpy(sc).cuda(), torch.from_numpy(bs).cuda(), p,
+                                  _dev(kw), inv_d, workspace=new_raw_workspace(step, "cuda"), rope_table=t).float())
+    a, b = outs
+    rel = float((a - b).norm() / b.norm())
+    print(f"[q8] table against own cos / sin, {pos + 1} rows: rel {rel:.2e}, {float((a != b).float().mean()):.2%} differ", flush=True)
+    assert rel <= 1e-3
