@@ -607,11 +607,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
         vec num = 0.0f;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
+            // (the operands selected, not the products: those stay fused into the sums)
             const bool live = mls[s][1] > 0.0f;
             const float w = live ? __builtin_amdgcn_exp2f(mls[s][0] - M) : 0.0f;
-            den += live ? mls[s][1] * w : 0.0f;
+            den = __builtin_fmaf(live ? mls[s][1] : 0.0f, w, den);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) num[e] += live ? w * a[s][e] : 0.0f;
+            for (int e = 0; e < VEC; ++e) num[e] = __builtin_fmaf(live ? a[s][e] : 0.0f, w, num[e]);
         }
         write(num * (1.0f / den));
         return;

@@ -140,6 +140,40 @@ def test_split_merge_counts(D, Hq, Hkv, Sq, Sk, split_keys):
                 seed=31 + D)
 
 
+@pytest.mark.parametrize("splits", [2, 4, 6, 8, 10])
+@pytest.mark.parametrize("D", [128, 512])
+def test_split_merge_rounds_once_per_split(D, splits):
+    """The merge alone, over partials written here: split 0 has the larger maximum (weight 1) and minus
+    the rounded product of split 1's sums and weight, so a fused multiply-add leaves that product's
+    rounding error and a separate product and sum exactly 0.  The weight is exp2(-0.5) to an ulp:
+    each third of the dims takes one of the three values, and none may be mostly zeros.  The other
+    splits are empty (l = 0) over sums that were never written."""
+    from apertura_amd.prefill import STAGE_MERGE, PrefillStep, prefill, prefill_workspace_bytes
+    Sk = 32 * splits
+    step = PrefillStep(1, 1, D, 1, Sk, Sk - 1, 0, split_keys=32)
+    assert prefill_workspace_bytes(step) == splits * (D * 4 + 8) + 256
+    rng = np.random.default_rng(17)
+    a1 = (1.0 + rng.random(D)).astype(np.float32)
+    w = np.float32(0.5 ** 0.5)
+    cand = np.array([np.nextafter(w, np.float32(0)), w, np.nextafter(w, np.float32(1))], dtype=np.float32)
+    acc = np.full((splits, D), np.nan, dtype=np.float32)
+    acc[0], acc[1] = -(a1 * cand[np.arange(D) % 3]), a1  # (numpy rounds the fp32 products)
+    ml = np.zeros((splits, 2), dtype=np.float32)
+    ml[:, 0] = -np.inf
+    ml[0], ml[1] = (0.0, 1.0), (-0.5, 1.0)
+    ws = torch.zeros(prefill_workspace_bytes(step), dtype=torch.uint8, device="cuda")
+    raw = np.concatenate([acc.reshape(-1), ml.reshape(-1)]).view(np.uint8)
+    ws[:raw.size] = torch.from_numpy(raw).cuda()
+    x = torch.zeros((1, Sk, D), dtype=torch.bfloat16, device="cuda")
+    out = prefill(step, x[:, :1], x, x, workspace=ws, stages=STAGE_MERGE)
+    torch.cuda.synchronize()
+    o = orc.from_bf16(_host(out)).reshape(D)
+    assert np.isfinite(o).all()
+    zeros = [float((o[c::3] == 0).mean()) for c in range(3)]
+    print(f"[prefill] merge of {splits} splits at {D}: zeros {zeros}, largest {np.abs(o).max():.1e}", flush=True)
+    assert max(zeros) < 0.5 and np.abs(o).max() <= 2.0 ** -22
+
+
 def test_split_merge_of_more_rows_than_a_launch_holds():
     """2^26 + 2^20 query rows at head dim 128 in three splits: the merge's wave per row is more threads
     than one launch takes.  Every head has the same query (head stride 0), so each position's
