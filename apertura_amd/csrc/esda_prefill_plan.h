@@ -57,10 +57,10 @@ ESDA_HD void tile_keys(const PrefillParams &p, int tile, int QT, int &j0, int &j
 // A kernel form of one head dim: 16-query blocks per wave, stage halves or not, waves, and
 // its cost in us: `wg` and `row` per workgroup and query row of it (Q and first-stage loads,
 // the pipeline's fill, epilogue) and `stage` per 32-key stage.  Fitted, with the split's costs
-// below, to graph-replayed times of 12,700 forced (form, split) plans of 1,230 chunks (1 .. 4096
-// queries, past 0 .. 16,000, GQA 1 .. 16, K = V or not); of the forced plans of a chunk the
-// cheapest by this cost then takes 1.008 (D = 128), 1.007 (256) and 1.013 (512) times the
-// fastest's time on average, 1.05, 1.05 and 1.06 at the 95th percentile.
+// below, to graph-replayed times of 20,000 forced (form, split) plans of 1,830 chunks (1 .. 4096
+// queries, past 0 .. 30,000, GQA 1 .. 16, K = V or not).  Of a chunk's forced plans the cheapest
+// by this cost then takes 1.008 (D = 128), 1.004 (256) and 1.010 (512) times the fastest's time
+// on average, 1.05, 1.03 and 1.06 at the 95th percentile, 1.20 at most.
 struct Tiling {
     int qb, kh, nw;
     float wg, row, stage;
@@ -73,13 +73,13 @@ struct Tiling {
 // eight on 128; but where CUs would idle, the smaller tiles halve what each loads and writes:
 // 32 fresh tokens 15.9 -> 10.1 us, 100 18.6 -> 13.0, 16 over 5016 keys 32.4 -> 28.7, 20 over 973
 // separate K / V rows 24.5 -> 21.3.
-constexpr Tiling kTilings512[] = {{1, 0, 8, 5.6f, 0.074f, 1.52f}, {1, 0, 4, 6.2f, 0.070f, 1.39f}};
-constexpr Tiling kTilings256[] = {{2, 0, 8, 7.0f, 0.037f, 1.457f}, {1, 0, 8, 5.0f, 0.037f, 0.95f},
-                                  {1, 1, 8, 6.0f, 0.049f, 0.6f}};
-constexpr Tiling kTilings128[] = {{2, 0, 8, 5.1f, 0.018f, 1.01f}};
+constexpr Tiling kTilings512[] = {{1, 0, 8, 5.7f, 0.076f, 1.54f}, {1, 0, 4, 6.2f, 0.066f, 1.6f}};
+constexpr Tiling kTilings256[] = {{2, 0, 8, 5.47f, 0.033f, 1.7f}, {1, 0, 8, 4.94f, 0.036f, 1.014f},
+                                  {1, 1, 8, 5.93f, 0.05f, 0.62f}};
+constexpr Tiling kTilings128[] = {{2, 0, 8, 5.16f, 0.017f, 1.055f}};
 
 constexpr int kXcds = 8, kEngines = 4, kEngineCus = kTargetGroups / (kXcds * kEngines);
-constexpr float kEmptyUs = 1.2f;  // a workgroup whose split holds no key of its tile
+constexpr float kEmptyUs = 1.0f;  // a workgroup whose split holds no key of its tile
 
 // Estimated us until the last workgroup of a plan ends.  Whatever their lengths, workgroup i
 // goes to XCD i % 8 and an XCD's workgroups in turn to its four engines of 8 CUs, each to the CU
@@ -121,7 +121,8 @@ inline float makespan(const Tiling &t, const int *nst, int tiles, int last_rows,
 // more: 32 MB 46.7 -> 45.7 us, 40 MB 43.7 both ways, 48 MB 42.2 -> 46.4, 64 MB 42.2 -> 54.0.
 constexpr float kPartNtBytes = 36.0e6f;
 inline float split_cost(float part_bytes, int splits) {  // us
-    return 3.0f + 2.2e-7f * part_bytes + 0.15f * std::max(0, splits - 8);
+    // (the merge's forms: up to 4 splits, up to 8, more)
+    return 3.2f + 2.2e-7f * part_bytes + (splits > 4 ? 0.3f : 0.0f) + (splits > 8 ? 0.9f + 0.11f * (splits - 8) : 0.0f);
 }
 constexpr int kMaxRounds = 3;  // split plans of more workgroups per CU only add partials
 

@@ -53,7 +53,7 @@ def _prefill_bytes(Hq, Hkv, D, Sq, Sk, q_pos0, k_pos0=0, window=0, split_keys=0)
     (32, 4, 512, 333, 5600, 3),    # 84 tiles of 4 heads: 252 workgroups, not 336
     (32, 4, 512, 200, 8056, 4),    # 52 tiles of 4 heads: 208
     (32, 4, 512, 512, 15872, 2),   # 128 tiles: 256
-    (32, 4, 512, 770, 0, 1),       # 388 fresh workgroups of four waves: unsplit
+    (32, 4, 512, 770, 0, 1),       # 49 fresh tiles of 4 heads: unsplit
     (32, 4, 512, 4096, 0, 1),      # four rounds of tiles
     (8, 4, 256, 17, 10, 1),        # one stage
 ])
@@ -121,7 +121,7 @@ def test_plans_follow_the_description_of_each_call(tmp_path):
 
     from apertura_amd import EsdaError
     base = dict(Hq=32, Hkv=4, D=512, Sq=200, Sk=8256, q_pos0=8056)
-    descs = [base, dict(base, Sq=199, q_pos0=8057), dict(base, split_keys=512), dict(base, window=1024),
+    descs = [base, dict(base, Sq=199, q_pos0=8057), dict(base, split_keys=512), dict(base, window=64),
              dict(base, D=256)]
     exe = _build(tmp_path, src=os.path.join(ROOT, "tests", "prefill_plan_check.cpp"))
     text = "".join(f"{d['Hq']} {d['Hkv']} {d['D']} {d['Sq']} {d['Sk']} {d['q_pos0']} 0 {d.get('window', 0)} "

@@ -225,7 +225,7 @@ PLANNED = [
     (512, 32, 4, 257, 700, 0, (8, 128, 3)),      # 17 tiles a head, the last of 8 rows: three splits fill one round
     (512, 16, 2, 16, 4900, 0, (4, 64, 31)),      # two 64-row tiles a head, many splits
     (512, 8, 8, 129, 0, 0, (4, 64, 1)),          # fresh, a last tile of one row
-    (512, 2, 1, 33, 3000, 0, (4, 64, 24)),       # two 64-row tiles, the last of two rows
+    (512, 2, 1, 33, 3000, 0, (4, 64, 32)),       # two 64-row tiles, the last of two rows
     (512, 32, 4, 600, 424, 0, (8, 128, 1)),      # 152 workgroups of eight waves, not 300 of four
     (256, 32, 16, 1100, 0, 256, (8, 128, 1)),    # 128-row tiles just past one round of the CUs
     (256, 16, 8, 17, 2000, 1024, (8, 128, 11)),  # one tile a head, splits
