@@ -611,9 +611,9 @@ void attend_kernel(AttendParams p) {
 //     one lane (k-steps 0, 1 and 8, 9); their bf16 cos / sin come from the table rows,
 //     whose buffer takes the next stage's table rows once the rotary k-steps have read it,
 //     or, when the caller passes no table, are computed by the lane that uses them (16 per
-//     lane and stage, ~430 VALU instructions: 131072 rows x 4 heads raw 105.7 us a step
-//     against 95.8 with the table and 160.6 by an 8-wave kernel that shared a computed
-//     table through LDS; q8 118.4, 95.3 and 207.5);
+//     lane and stage, about 500 VALU instructions: 131072 rows x 4 heads raw 104 us a step
+//     against 95 with the table and 164 by an 8-wave kernel that shared a computed table
+//     through LDS; q8 118, 96 and 207);
 //   - scores the kv head's query heads (up to 16: the MFMA's N dimension, zero-padded) with
 //     16 MFMAs, runs its own online softmax, and accumulates O^T[512 x 16 heads] with 32
 //     MFMAs over V = kraw read back by transpose reads, rinv folded into the weight:
@@ -1007,7 +1007,7 @@ void raw_attend_kernel(AttendParams p) {
                     fq = bias * rinv;
                     // Without a table both quotients are IEEE divisions: within half an ulp each, where
                     // the reciprocal instruction is within one (~25 more VALU instructions a stage
-                    // beside the ~430 of the cos / sin).
+                    // beside the ~500 of the cos / sin).
                     if (lg == 0) {
                         xfw[0 * 16 + li] = rq;
                         xfw[1 * 16 + li] = TABLE ? __builtin_amdgcn_rcpf(rq) : 1.0f / rq;
@@ -1447,7 +1447,7 @@ __global__ __launch_bounds__(kMergeRowsThreads) void merge_rows_kernel(MergePara
 
 // Per-row affine u8 of raw rows (esQuantizeRawRows, ESDecodeAttn.mm:491-539): one wave
 // per row of src [kv heads, n, 512] bf16; row (h, i) -> q8[h * q_head_stride + (row0 + i)
-// * 512 ..], scale / bias at [h * sb_head_stride + row0 + i].  The attend kernel's q8 mode
+// * 512 ..], scale / bias at [h * sb_head_stride + row0 + i].  raw_attend_kernel's q8 form
 // quantizes the decode step's new row with the same arithmetic.
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint16_t *src, int n, long long rows,
                                                             unsigned char *q8, long long q_head_stride,

@@ -24,11 +24,13 @@
 //                       straight from the score registers (the 32 keys are ordered so
 //                       that the score layout is the B-operand layout).  O^T stays in
 //                       registers (D/16 x QB tiles: QB * D / 16 accumulators per lane).
-//                       Four waves and 64-row tiles for short chunks at D = 512.
+//                       Four waves and 64-row tiles at D = 512 where the plan
+//                       (esda_prefill_plan.h) finds them faster: mostly chunks whose 128-row
+//                       tiles would leave CUs idle.
 //   prefill_kernel<256, 1, true>  the same with 64-row tiles whose even and odd stages go
 //                       to the two wave groups (waves 0-3 and 4-7 on the same query
-//                       blocks), folded together through LDS at the end: short chunks
-//                       at D = 256 fill the CUs with tiles instead of key splits.
+//                       blocks), folded together through LDS at the end: chunks whose
+//                       128-row tiles would leave CUs idle at D = 256.
 //   prefill_merge_kernel  reduces split partials (m, l, acc) per (query row, head).
 //   raw_prefill_kv_kernel rebuilds K and V of a raw-K (or q8 raw-K) stream by the
 //                       reference's op-level rounding points.
