@@ -217,8 +217,13 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
                 const float spread = even + (float) (pieces - tiles) * d->num_kv_heads * t.wg / kTargetGroups;
                 if (us + std::max(spread, rounds * (t.wg + per * t.stage)) >= best) return;
                 us += makespan(t, nst, (int) tiles, last_rows, d->num_kv_heads, splits, per);
-            } else {  // many workgroups: the CUs stay busy but for the end of the last round
-                us += even + 0.5f * (t.wg + t.row * QT + most * t.stage);
+            } else {
+                // many workgroups (many tiles, or forced splits of any count): each piece starts anew, and
+                // the CUs stay busy but for the end of the last round.  (70 chunks of forced splits that
+                // took shorter tiles without the pieces' starts: 14% less time on average; 3028 queries
+                // over 3787 keys in 4 splits, D = 256, 16 heads, 344 us in 128-row tiles, 229 in 256-row.)
+                const double more = (double) tiles * (splits - 1) * d->num_kv_heads / kTargetGroups;
+                us += even + (float) more * (t.wg + t.row * QT) + 0.5f * (t.wg + t.row * QT + std::min(per, most) * t.stage);
             }
             if (us < best) {
                 best = us;

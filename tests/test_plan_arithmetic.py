@@ -114,6 +114,14 @@ def test_prefill_forms_the_planned_tests_rely_on(tmp_path):
     assert _plans(tmp_path, [(32, 8, 128, 2043, 0, 0, 0), (16, 16, 512, 1364, 91, 0, 0)]) == [(8, 256, 1), (4, 64, 1)]
 
 
+def test_forced_splits_of_many_workgroups_take_tall_tiles(tmp_path):
+    """Forced splits past three workgroups a CU: every piece loads its queries and fills its pipeline
+    anew, so the tall tiles, which have fewer pieces, are the cheap ones."""
+    chunks = [(32, 16, 256, 3028, 759, 0, 1024), (16, 8, 256, 2005, 0, 0, 512), (8, 4, 256, 3163, 954, 0, 256),
+              (8, 1, 256, 2091, 36, 1024, 128), (16, 2, 512, 969, 0, 0, 128)]
+    assert _plans(tmp_path, chunks) == [(8, 256, 4), (8, 256, 4), (8, 256, 17), (8, 256, 9), (8, 128, 8)]
+
+
 def test_plans_follow_the_description_of_each_call(tmp_path):
     """The library keeps the calling thread's last plan: descriptions that differ in one field, taken
     in turn and from two threads at once, get their own workspace sizes, refused ones none."""
