@@ -562,14 +562,18 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_kernel(PrefillParams p) {
 // l_s > 0.  One wave per (row, 64 * VEC dims).  Memory-bound: splits * D * 4 bytes per row,
 // read once, so the two forms differ in how they cover the latency:
 //  - NS > 0, for plans of at most NS splits: every (m, l) and partial row is loaded at once
-//    (one round trip; a row that an empty split never wrote is dropped by a select);
+//    (one round trip; a row that an empty split never wrote is dropped by a select), or with
+//    GAPS, where the plan leaves many tiles' last splits empty, the (m, l) and then the live
+//    splits' rows: a fresh prompt's rows see the splits up to their own, a little over half of
+//    them (2048 queries of 32 heads in 4 splits, D = 512, 0.54 GB: 116 us reading all, 75 the
+//    live ones; 805 MB in 6, 174 and 114);
 //  - NS = 0: lane j loads (m, l) of split j (and j + 64, ..), so the max, the weights and the
 //    denominator take one round trip and wave reductions, and the wave then walks the live
 //    splits (a ballot: wave-uniform) with MB of their rows in flight.
 // A thread per 4 dims walking the splits one after another was bound by their latency:
 // 512 rows of D = 512 with 18 splits 8.2 us against 4.3 here, with 32 splits 19.9 against
 // 6.3; 16384 rows with 2 splits 17.2 against 14.4 (67 MB at 4.7 TB/s).
-template <int D, int NS>
+template <int D, int NS, bool GAPS = false>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     constexpr int VEC = D >= 256 ? 4 : D / 64;  // dims per lane
     constexpr int PARTS = D / (64 * VEC);       // waves per row
@@ -600,8 +604,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
             a[s] = 0.0f;
             if (s < p.splits) {
                 mls[s] = *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * ((long long) s * nrows + row));
-                a[s] = *reinterpret_cast<const vec *>(acc + s * ss);
+                if (!GAPS) a[s] = *reinterpret_cast<const vec *>(acc + s * ss);
             }
+        }
+        if (GAPS) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                if (mls[s][1] > 0.0f) a[s] = *reinterpret_cast<const vec *>(acc + s * ss);
         }
         float M = -INFINITY, den = 0.0f;
 #pragma unroll
@@ -857,7 +866,9 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
         for (mp.merge_wave0 = 0; mp.merge_wave0 < waves; mp.merge_wave0 += kMergeLaunchWaves) {
             const long long n = std::min(kMergeLaunchWaves, waves - mp.merge_wave0);
             const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
-            if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, mp);
+            if (p.part_gaps && p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4, true>), grid, block, 0, st, mp);
+            else if (p.part_gaps && p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8, true>), grid, block, 0, st, mp);
+            else if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, mp);
             else if (p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8>), grid, block, 0, st, mp);
             else hipLaunchKernelGGL((prefill_merge_kernel<D, 0>), grid, block, 0, st, mp);
         }

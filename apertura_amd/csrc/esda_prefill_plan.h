@@ -31,6 +31,7 @@ struct PrefillParams {
     int kh;                  // 1: the two wave groups split each tile's stages (even / odd)
     int nw;                  // waves per workgroup (query tile: 16 qb nw rows, half of it with kh)
     int part_nt;             // 1: partials stored non-temporal
+    int part_gaps;           // 1: the merge reads the partials of live splits only
     long long merge_wave0;   // the split merge's launch: its first wave
 };
 
@@ -120,6 +121,13 @@ inline float makespan(const Tiling &t, const int *nst, int tiles, int last_rows,
 // L2s together (8 x 4 MB) the write-back overlaps the kernel, and waiting for memory costs
 // more: 32 MB 46.7 -> 45.7 us, 40 MB 43.7 both ways, 48 MB 42.2 -> 46.4, 64 MB 42.2 -> 54.0.
 constexpr float kPartNtBytes = 36.0e6f;
+
+// Where a quarter of the tiles have no key in the last split (the first ones: a tile sees more
+// than those before it, up to the window), the merge first reads which splits of a row are
+// live.  That second round trip costs few partials more than their empty ones do: fresh queries
+// of 16 heads, D = 256, 8.4 MB (256 in 2 splits) 2.8 -> 3.1 us, 12.6 MB 3.2 -> 3.5, 16.8 MB
+// 3.6 -> 3.6 .. 4.2, 25 MB 5.0 -> 4.9, 50 MB 9.0 -> 6.1.
+constexpr float kGapBytes = 20.0e6f;
 inline float split_cost(float part_bytes, int splits) {  // us
     // (the merge's forms: up to 4 splits, up to 8, more)
     return 3.2f + 2.2e-7f * part_bytes + (splits > 4 ? 0.3f : 0.0f) + (splits > 8 ? 0.9f + 0.11f * (splits - 8) : 0.0f);
@@ -254,7 +262,11 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
         return "esda_prefill: too many key splits";
     p->kps = kps;
     p->splits = (int) std::max<long long>(1, splits);
-    p->part_nt = 4.0f * D * p->Sq * p->Hq * p->splits <= kPartNtBytes;
+    const float part_bytes = 4.0f * D * p->Sq * p->Hq * p->splits;
+    p->part_nt = part_bytes <= kPartNtBytes;
+    int a, b;
+    tile_keys(*p, p->tiles / 4, 16 * p->qb * (p->kh ? p->nw / 2 : p->nw), a, b);
+    p->part_gaps = part_bytes > kGapBytes && b - a <= (p->splits - 1) * (long long) p->kps;
     return nullptr;
 }
 

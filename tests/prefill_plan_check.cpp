@@ -1,7 +1,8 @@
 // prefill_plan_check.cpp -- the plan of esda_prefill (apertura_amd/csrc/esda_prefill_plan.h)
 // for descriptions read from standard input, one per line: "Hq Hkv D Sq Sk q_pos0 k_pos0
 // window split_keys".  Prints, per line, the kernel form and split (waves, query rows per
-// tile, tiles per kv head, key splits, keys per split, workspace bytes), or the refusal.
+// tile, tiles per kv head, key splits, keys per split, whether the merge reads live splits
+// only, workspace bytes), or the refusal.
 // Built and run by tests/test_plan_arithmetic.py with g++.
 #include "esda_prefill_plan.h"
 
@@ -21,8 +22,8 @@ int main() {
         esda_prefill_plan::PrefillParams p;
         if (const char *why = esda_prefill_plan::plan_prefill(&d, &p)) std::printf("refused: %s\n", why);
         else
-            std::printf("%d %d %d %d %d %zu\n", p.nw, 16 * p.qb * (p.kh ? p.nw / 2 : p.nw), p.tiles, p.splits, p.kps,
-                        esda_prefill_plan::workspace_of(p, d.head_dim));
+            std::printf("%d %d %d %d %d %d %zu\n", p.nw, 16 * p.qb * (p.kh ? p.nw / 2 : p.nw), p.tiles, p.splits, p.kps,
+                        p.part_gaps, esda_prefill_plan::workspace_of(p, d.head_dim));
         ++n;
     }
     return n == 0;

@@ -78,9 +78,10 @@ def test_prefill_plan_of_extreme_forced_splits_is_quick():
     assert time.perf_counter() - t0 < 2.0
 
 
-def _plans(tmp_path, descs):
+def _plans(tmp_path, descs, gaps=False):
     """The plans of (Hq, Hkv, D, Sq, past, window, split_keys), the chunk's own keys and its past (on
-    sliding layers the last window of it): (waves, rows per tile, splits) each, or the refusal."""
+    sliding layers the last window of it): (waves, rows per tile, splits) each, with gaps also whether
+    the merge reads live splits only, or the refusal."""
     exe = _build(tmp_path, src=os.path.join(ROOT, "tests", "prefill_plan_check.cpp"))
     lines = []
     for Hq, Hkv, D, Sq, past, window, split in descs:
@@ -93,8 +94,8 @@ def _plans(tmp_path, descs):
         if line.startswith("refused"):
             out.append(line)
         else:
-            nw, qt, tiles, splits, kps, nbytes = map(int, line.split())
-            out.append((nw, qt, splits))
+            nw, qt, tiles, splits, kps, live_only, nbytes = map(int, line.split())
+            out.append((nw, qt, splits, live_only) if gaps else (nw, qt, splits))
     return out
 
 
@@ -120,6 +121,16 @@ def test_forced_splits_of_many_workgroups_take_tall_tiles(tmp_path):
     chunks = [(32, 16, 256, 3028, 759, 0, 1024), (16, 8, 256, 2005, 0, 0, 512), (8, 4, 256, 3163, 954, 0, 256),
               (8, 1, 256, 2091, 36, 1024, 128), (16, 2, 512, 969, 0, 0, 128)]
     assert _plans(tmp_path, chunks) == [(8, 256, 4), (8, 256, 4), (8, 256, 17), (8, 256, 9), (8, 128, 8)]
+
+
+def test_merges_that_read_live_splits_only(tmp_path):
+    """Where a large split plan leaves a quarter of the tiles without a key in the last split: fresh
+    prompts, not small ones, nor a past or a window that fills all splits but the last."""
+    from test_prefill_gpu import GAPS
+    plans = _plans(tmp_path, [(Hq, Hkv, D, Sq, past, window, split) for D, Hq, Hkv, Sq, past, window, split, _ in GAPS], gaps=True)
+    assert [(s, g) for _, _, s, g in plans] == [(s, 1) for *_, s in GAPS]
+    same = [(32, 4, 512, 512, 8192, 0, 1088), (16, 8, 256, 256, 0, 0, 128), (16, 8, 256, 2048, 9000, 1024, 512)]
+    assert [p[2:] for p in _plans(tmp_path, same, gaps=True)] == [(8, 0), (2, 0), (3, 0)]
 
 
 def test_plans_follow_the_description_of_each_call(tmp_path):

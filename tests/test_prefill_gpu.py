@@ -174,6 +174,32 @@ def test_split_merge_rounds_once_per_split(D, splits):
     assert max(zeros) < 0.5 and np.abs(o).max() <= 2.0 ** -22
 
 
+# Merges that read live splits only: D, query heads, kv heads, queries, past, window, split_keys, splits.
+GAPS = [(512, 4, 4, 701, 0, 0, 192, 4), (512, 4, 1, 389, 500, 0, 128, 7), (256, 7, 7, 1001, 0, 0, 352, 3),
+        (256, 3, 3, 2003, 0, 1024, 320, 4), (128, 5, 5, 1667, 0, 0, 288, 6), (128, 5, 1, 5003, 0, 0, 2528, 2)]
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,Sq,past,window,split_keys,splits", GAPS)
+def test_split_merge_of_live_splits(D, Hq, Hkv, Sq, past, window, split_keys, splits):
+    """Empty splits of early rows, whose partials are NaN before the call."""
+    from apertura_amd.prefill import PrefillStep, prefill, prefill_workspace_bytes
+    rng = np.random.default_rng(29)
+    Sk = past + Sq
+    q, k, v = rms_rows(rng, (Hq, Sq, D)), rms_rows(rng, (Hkv, Sk, D)), rms_rows(rng, (Hkv, Sk, D))
+    step = PrefillStep(Hq, Hkv, D, Sq, Sk, past, 0, window, scale=D ** -0.5, split_keys=split_keys)
+    assert prefill_workspace_bytes(step) == splits * Sq * Hq * (D * 4 + 8) + 256
+    ws = torch.full((prefill_workspace_bytes(step),), 255, dtype=torch.uint8, device="cuda")
+    out = prefill(step, _dev(q), _dev(k), _dev(v), workspace=ws)
+    torch.cuda.synchronize()
+    o = orc.from_bf16(_host(out)).astype(np.float64)
+    worst = 0.0
+    for r0 in list(range(0, Sq, 97)) + [Sq - 1]:
+        ref = orc.prefill_f64(q[:, r0:r0 + 1], k, v, past + r0, 0, window, D ** -0.5)
+        worst = max(worst, float(np.abs(o[r0:r0 + 1] - ref).max()))
+    print(f"[prefill] live splits D={D} Sq={Sq}: max_abs={worst:.3e}", flush=True)
+    assert np.isfinite(o).all() and worst <= TOL_MAX
+
+
 def test_split_merge_of_more_rows_than_a_launch_holds():
     """2^26 + 2^20 query rows at head dim 128 in three splits: the merge's wave per row is more threads
     than one launch takes.  Every head has the same query (head stride 0), so each position's
