@@ -559,7 +559,8 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_kernel(PrefillParams p) {
 }
 
 // out(i, h, :) = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the splits with
-// l_s > 0.  One wave per (row, 64 * VEC dims).  Memory-bound: splits * D * 4 bytes per row,
+// l_s > 0.  One wave per (row, 64 * VEC dims), or per two rows of 128 dims (in up to 8 splits).
+// Memory-bound: splits * D * 4 bytes per row,
 // read once, so the two forms differ in how they cover the latency:
 //  - NS > 0, for plans of at most NS splits: every (m, l) and partial row is loaded at once
 //    (one round trip; a row that an empty split never wrote is dropped by a select), or with
@@ -572,20 +573,23 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_kernel(PrefillParams p) {
 //    splits (a ballot: wave-uniform) with MB of their rows in flight.
 // A thread per 4 dims walking the splits one after another was bound by their latency:
 // 512 rows of D = 512 with 18 splits 8.2 us against 4.3 here, with 32 splits 19.9 against
-// 6.3; 16384 rows with 2 splits 17.2 against 14.4 (67 MB at 4.7 TB/s).
+// 6.3; 16384 rows with 2 splits 17.2 against 14.4 (67 MB at 4.7 TB/s).  A wave per row of 128
+// dims, 2 a lane, had too few bytes in flight for many rows: 16,384 rows with 2 splits 6.9 us
+// against 5.4 here, 32,768 10.9 against 9.3.
 template <int D, int NS, bool GAPS = false>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
-    constexpr int VEC = D >= 256 ? 4 : D / 64;  // dims per lane
-    constexpr int PARTS = D / (64 * VEC);       // waves per row
+    constexpr int VEC = D >= 256 || NS > 0 ? 4 : D / 64;              // dims per lane
+    constexpr int LPR = D / VEC < 64 ? D / VEC : 64, RPW = 64 / LPR;  // lanes per row and wave, rows per wave
+    constexpr int PARTS = D / (LPR * VEC);                            // waves per row
     constexpr int MB = 8;                       // partial rows in flight
     typedef float vec __attribute__((ext_vector_type(VEC)));
     typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
     const int lane = threadIdx.x & 63;
     const long long nrows = (long long) p.Sq * p.Hq;
     const long long wv = p.merge_wave0 + (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
-    if (wv >= nrows * PARTS) return;
-    const long long row = wv / PARTS;
-    const int d0 = (int) (wv % PARTS) * 64 * VEC + lane * VEC;
+    const long long row = RPW * (wv / PARTS) + (RPW > 1 ? lane / LPR : 0);
+    if (row >= nrows) return;
+    const int d0 = (int) (wv % PARTS) * 64 * VEC + lane % LPR * VEC;
     const float *acc = p.part_acc + row * D + d0;
     const long long ss = nrows * D;
     auto write = [&](const vec &v) {

@@ -270,10 +270,13 @@ inline const char *plan_prefill(const esda_prefill_desc *d, PrefillParams *p) {
     return nullptr;
 }
 
-// Waves of the split merge: one per query row of up to 256 dims, and as many as a launch takes
-// (2^31 threads; a HIP launch holds fewer than 2^32).  More rows take several launches.
+// A launch of the split merge takes 2^31 threads (a HIP launch holds fewer than 2^32).  More rows
+// take several.
 constexpr long long kMergeLaunchWaves = 1LL << 25;
-inline long long merge_waves(const PrefillParams &p, int D) { return (long long) p.Sq * p.Hq * (D == 512 ? 2 : 1); }
+inline long long merge_waves(const PrefillParams &p, int D) {
+    const long long rows = (long long) p.Sq * p.Hq;
+    return D == 512 ? 2 * rows : D == 128 && p.splits <= 8 ? (rows + 1) / 2 : rows;
+}
 
 inline size_t workspace_of(const PrefillParams &p, int D) {
     if (p.splits <= 1) return 0;

@@ -201,7 +201,7 @@ def test_split_merge_of_live_splits(D, Hq, Hkv, Sq, past, window, split_keys, sp
 
 
 def test_split_merge_of_more_rows_than_a_launch_holds():
-    """2^26 + 2^20 query rows at head dim 128 in three splits: the merge's wave per row is more threads
+    """2^26 + 2^20 query rows at head dim 128 in three splits: the merge's wave per two rows is more threads
     than one launch takes.  Every head has the same query (head stride 0), so each position's
     output is checked once against the oracle and every head against the first."""
     from apertura_amd.prefill import PrefillStep, prefill, prefill_workspace_bytes
