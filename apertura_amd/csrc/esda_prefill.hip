@@ -559,9 +559,11 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_kernel(PrefillParams p) {
 }
 
 // out(i, h, :) = sum_s acc_s 2^(m_s - M) / sum_s l_s 2^(m_s - M) over the splits with
-// l_s > 0.  One wave per (row, 64 * VEC dims), or per two rows of 128 dims (in up to 8 splits).
-// Memory-bound: splits * D * 4 bytes per row,
-// read once, so the two forms differ in how they cover the latency:
+// l_s > 0.  One wave per (row, 64 * VEC dims), or per two rows of 128 dims (in up to 8 splits; a
+// block is then two waves, since four rows a block keep a GQA group of four on the XCD that
+// wrote it: 143 queries of 32 heads over 8 in 8 splits, 4.1 us and 5.9 with eight rows a block).
+// Memory-bound: splits * D * 4 bytes per row, read once, so the two forms differ in how they
+// cover the latency:
 //  - NS > 0, for plans of at most NS splits: every (m, l) and partial row is loaded at once
 //    (one round trip; a row that an empty split never wrote is dropped by a select), or with
 //    GAPS, where the plan leaves many tiles' last splits empty, the (m, l) and then the live
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     typedef __bf16 bvec __attribute__((ext_vector_type(VEC)));
     const int lane = threadIdx.x & 63;
     const long long nrows = (long long) p.Sq * p.Hq;
-    const long long wv = p.merge_wave0 + (long long) blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+    const long long wv = p.merge_wave0 + (long long) blockIdx.x * (4 / RPW) + uniform(threadIdx.x >> 6);
     const long long row = RPW * (wv / PARTS) + (RPW > 1 ? lane / LPR : 0);
     if (row >= nrows) return;
     const int d0 = (int) (wv % PARTS) * 64 * VEC + lane % LPR * VEC;
@@ -869,7 +871,8 @@ void launch_prefill(const PrefillParams &p, int stages, hipStream_t st) {
         PrefillParams mp = p;
         for (mp.merge_wave0 = 0; mp.merge_wave0 < waves; mp.merge_wave0 += kMergeLaunchWaves) {
             const long long n = std::min(kMergeLaunchWaves, waves - mp.merge_wave0);
-            const dim3 grid((unsigned) ((n + 3) / 4)), block(256);
+            const int wpb = D == 128 && p.splits <= 8 ? 2 : 4;  // waves per block: the kernel's 4 / RPW
+            const dim3 grid((unsigned) ((n + wpb - 1) / wpb)), block(64 * wpb);
             if (p.part_gaps && p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4, true>), grid, block, 0, st, mp);
             else if (p.part_gaps && p.splits <= 8) hipLaunchKernelGGL((prefill_merge_kernel<D, 8, true>), grid, block, 0, st, mp);
             else if (p.splits <= 4) hipLaunchKernelGGL((prefill_merge_kernel<D, 4>), grid, block, 0, st, mp);
