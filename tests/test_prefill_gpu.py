@@ -273,6 +273,15 @@ def test_planned_forms_and_splits(D, Hq, Hkv, Sq, past, window, form):
                 window=window, seed=51, rows=rows, shared=D == 512 and Hkv == 4)
 
 
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,Sq,past,split_keys", [(2, 2, 1, 0, 0), (4, 1, 16, 1500, 0), (3, 1, 21, 33, 32), (8, 1, 8, 600, 0),
+                                                       (5, 5, 65, 300, 64)])
+def test_one_tile_at_512_goes_by_the_streams(Hq, Hkv, Sq, past, split_keys, shared):
+    """Up to 64 rows a kv head (63, 64, and 65 past it): four waves with one K = V buffer, eight without."""
+    run_prefill(f"tile-{Sq * Hq // Hkv}-{int(shared)}", Hq=Hq, Hkv=Hkv, D=512, Sq=Sq, Sk=past + Sq, q_pos0=past, k_pos0=0,
+                seed=53, shared=shared, split_keys=split_keys)
+
+
 def test_local_sliding_window_with_evicted_keys():
     # chunked prefill keeps window + seq keys (ESAttention.mm:99-103): pastLen 500
     run_prefill("local-window", Hq=8, Hkv=4, D=256, Sq=200, Sk=264, q_pos0=500, k_pos0=436, window=64, seed=3)
