@@ -309,7 +309,7 @@ def decode_raw(step: RawStep, q: torch.Tensor, k_new: torch.Tensor | None, raw_c
                stages: int = STAGE_ATTEND | STAGE_MERGE, rope_table: torch.Tensor | None = None) -> torch.Tensor:
     """Raw-K decode step: write k_new (raw rows, or None) at row pos[b], then attend rows
     0 .. pos[b]; returns out [B, Hq, 512] bf16.  rope_table: an optional precomputed
-    rotary table (rope_table(), >= cap rows), bit-identical to the kernel's own."""
+    rotary table (rope_table(), >= cap rows), whose values are the ones computed without it."""
     bf = torch.bfloat16
     if q.shape != (step.batch, step.num_q_heads, 512) or not q.is_contiguous():
         raise ValueError("q must be contiguous [B, Hq, 512]")

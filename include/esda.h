@@ -177,7 +177,9 @@ int esda_decode_raw_workspace_size(const esda_raw_desc *desc, size_t *bytes);
  * (ESDecodeAttn.mm:415-453) as called at ESAttention.mm:291-300. */
 int esda_decode_raw(const esda_raw_desc *desc, const esda_raw_args *args, void *stream);
 
-/* Stage-selectable form of esda_decode_raw (ESDA_STAGE_* as for esda_decode_stages). */
+/* Stage-selectable form of esda_decode_raw (ESDA_STAGE_* as for esda_decode_stages).  Stages
+ * launched separately take the same arguments: the merge's shares depend on whether
+ * rope_table is set. */
 int esda_decode_raw_stages(const esda_raw_desc *desc, const esda_raw_args *args, int stages,
                            void *stream);
 
